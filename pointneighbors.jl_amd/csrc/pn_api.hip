@@ -173,7 +173,6 @@ int pn_grid_refresh(pn_grid_t grid, const void* y, int64_t n_y) {
     BinSet& s = grid->grid;
     if (!s.valid) return fail(PN_ERR_NOT_INITIALIZED, "the neighborhood search is not initialized");
     if (n_y != s.n_src) return fail(PN_ERR_ARGUMENT, "coordinate matrix size differs from the last update!");
-    ++grid->gen;  // coordinates changed: recorded pair lists are stale
     s.fresh = false;  // and so are a hash grid's per-bucket cells
     if (s.n_sel == 0) return PN_OK;
     return dispatch_build(*grid, [&](auto dc, auto tcv, auto) -> int {
@@ -352,13 +351,11 @@ int pn_set_tuning(pn_grid_t grid, const char* key, int64_t value) {
     if (k == "chunk") {
         if (value < -1 || value > 1) return fail(PN_ERR_ARGUMENT, "chunk must be -1, 0 or 1");
         grid->chunk = (int)value;
-        grid->pc_gen = ~0ull;
         return PN_OK;
     }
     if (k == "algorithm") {
         if (value != 0 && value != 1) return fail(PN_ERR_ARGUMENT, "algorithm must be 0 or 1");
         grid->algorithm = (int)value;
-        grid->pc_gen = ~0ull;
         return PN_OK;
     }
     if (k == "time_launches") {
@@ -367,16 +364,12 @@ int pn_set_tuning(pn_grid_t grid, const char* key, int64_t value) {
         grid->timing_used = 0;
         return PN_OK;
     }
-    if (k == "pair_cache") {
+    if (k == "pair_cache") {  // accepted without effect
         if (value != 0 && value != 1) return fail(PN_ERR_ARGUMENT, "pair_cache must be 0 or 1");
-        grid->pair_cache = (int)value;
-        grid->pc_gen = ~0ull;
         return PN_OK;
     }
-    if (k == "pair_cache_per_point") {
+    if (k == "pair_cache_per_point") {  // accepted without effect
         if (value < 0) return fail(PN_ERR_ARGUMENT, "pair_cache_per_point must be >= 0");
-        grid->pc_per_point = value;
-        grid->pc_gen = ~0ull;
         return PN_OK;
     }
     if (k == "canonical_order") {

@@ -164,16 +164,17 @@ int pn_count_neighbors_noalloc(int ndims, int coord_dtype, int radius_dtype, int
         hipLaunchKernelGGL((pn::k_canon<D, TC>), dim3(blocks_for(n, 256)), dim3(256), 0, s, (const int32_t*)keys,
                            (int64_t)0, (const int32_t*)nullptr, (const pn::DevStatus*)st, (const int32_t*)start,
                            (const int32_t*)perm_tmp, (const TC*)y, sorted_idx, (TC*)coords, std::max<int64_t>(n, 1),
-                           1);
+                           1, slots);
         PN_CHECK_LAUNCH();
         return PN_OK;
     });
     if (rc) return rc;
 
-    // count: the cell traversal of pn_count_neighbors over the grid's own points
+    // count: the traversal of pn_count_neighbors over the grid's own points
     pn::SetView v;
     v.start = start;
     v.nonempty = nonempty;
+    v.keys = slots;
     v.sorted_idx = sorted_idx;
     v.coords = coords;
     v.cap = std::max<int64_t>(n, 1);
@@ -181,15 +182,24 @@ int pn_count_neighbors_noalloc(int ndims, int coord_dtype, int radius_dtype, int
     pn::CountF f;
     f.out = counts;
     f.accumulate = 0;
-    const int nblocks = (int)std::min<int64_t>(round_up8(std::min<int64_t>(C, n)), int64_t(1) << 20);
+    const bool runs = runs_apply<pn::CountF>(g);
+    pn::RunScale sc;
+    pn::RunSplit sp;
+    run_params(g, n, false, true, true, sc, sp);
+    const int64_t nwork = runs ? (n + sp.most - 1) / sp.most : std::min<int64_t>(C, n);
+    const int nblocks = (int)std::min<int64_t>(round_up8(nwork), int64_t(1) << 20);
     rc = dispatch_trav(g, [&](auto dc, auto tcv, auto trv) -> int {
         constexpr int D = decltype(dc)::value;
         using TC = decltype(tcv);
         using TR = decltype(trv);
         constexpr int G = pn::CellGroups<TC, pn::CountF>::large;
         const TR r = (TR)search_radius;
-        hipLaunchKernelGGL((pn::k_cells<D, TC, TR, pn::CountF, G, false, 0>), dim3(nblocks), dim3(pn::WAVE), 0, s,
-                           g.geom, v, v, r * r, f, nblocks, pn::PairCache{});
+        if (runs)
+            hipLaunchKernelGGL((pn::k_runs_count<D, TC, TR, false>), dim3(nblocks), dim3(pn::WAVE), 0, s, g.geom, v, v,
+                               r * r, f, nblocks, sc, sp);
+        else
+            hipLaunchKernelGGL((pn::k_cells<D, TC, TR, pn::CountF, G, false>), dim3(nblocks), dim3(pn::WAVE), 0, s,
+                               g.geom, v, v, r * r, f, nblocks);
         PN_CHECK_LAUNCH();
         return PN_OK;
     });

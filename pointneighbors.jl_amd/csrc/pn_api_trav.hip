@@ -44,7 +44,8 @@ int pn_csr_count(pn_grid_t grid, int queries, int64_t n_rows, int32_t* row_ptr, 
     pn::CountF f;
     f.out = g.csr_counts.as<int32_t>();
     f.accumulate = 0;
-    if ((rc = launch_traverse(g, queries, f))) return rc;
+    // lists are mostly made of undeformed lattices, whose ties the cell kernel counts faster
+    if ((rc = launch_traverse(g, queries, f, false))) return rc;
     if ((rc = g.csr_scan.run(g.csr_counts.as<int32_t>(), n_rows, row_ptr, nullptr, st, g.stream))) return rc;
     PN_HIP(hipMemcpyAsync(g.csr_host_status, st, sizeof(pn::DevStatus), hipMemcpyDeviceToHost, g.stream));
     PN_HIP(hipStreamSynchronize(g.stream));

@@ -96,6 +96,7 @@ struct SetView {
     const int32_t* start;       // C + 1 cell offsets
     const int32_t* nonempty;    // non-empty cell ids
     const int32_t* sorted_idx;  // original index per sorted position
+    const int32_t* keys;        // cell per sorted position (NULL for a SpatialHashingCellList)
     const void* coords;         // D planes of cap entries, cell-sorted
     int64_t cap;
     const DevStatus* st;
@@ -475,8 +476,8 @@ constexpr int CANON_RANK_LIMIT = 1024;
 // and repeated selections of one point get distinct consecutive slots), or k itself
 // (canonical = 0: the order of the reference's ParallelUpdate, nondeterministic inside a
 // cell; neighbour sets are the same).  A wavefront's stores land inside the cell segments
-// of its 64 slots, so the permutation and the cell-sorted coordinate planes (plane d at
-// coords + d * cap) are written in whole lines.
+// of its 64 slots, so the permutation, the cell per sorted position and the cell-sorted
+// coordinate planes (plane d at coords + d * cap) are written in whole lines.
 // Slot k's canonical position pos, its selection position a, point p, cell key and the first
 // slot s of the cell segment.
 struct CanonSlot {
@@ -517,11 +518,13 @@ __global__ __launch_bounds__(256) void k_canon(const int32_t* __restrict__ keys,
                                                const int32_t* __restrict__ start,
                                                const int32_t* __restrict__ perm_tmp,
                                                const TC* __restrict__ y, int32_t* __restrict__ sorted_idx,
-                                               TC* __restrict__ coords, int64_t cap, int canonical) {
+                                               TC* __restrict__ coords, int64_t cap, int canonical,
+                                               int32_t* __restrict__ sorted_keys) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= st->n_binned) return;
     const CanonSlot c = canon_slot(keys, sel_first, sel_list, start, perm_tmp, k, canonical);
     sorted_idx[c.pos] = c.p;
+    sorted_keys[c.pos] = c.key;
 #pragma unroll
     for (int d = 0; d < D; ++d) coords[(int64_t)d * cap + c.pos] = y[(int64_t)D * c.p + d];
 }

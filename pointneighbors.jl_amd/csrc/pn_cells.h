@@ -28,21 +28,6 @@ namespace pn {
 // Pair-list capacity (entries) of the candidate-major traversal.
 constexpr int PAIR_CAP = 1024;
 
-// Pair cache: the first traversal of a cacheable functor after a build records, per
-// non-empty cell, its flushes; later traversals on the same build replay them instead of
-// testing candidates.  Each wavefront appends the records of its cells to its own region
-// of `data` (no atomics); a cell's records are contiguous:
-//     record = [batch, chunk, i0, i1, qstart[0 .. i1-i0], pair[0 .. P-1]]   (P = qstart[i1-i0])
-// head[2w] = first entry / 4 of work item w's records (-1: not cached, the replay runs
-// the full traversal for it), head[2w+1] = their length.  A replay loads a cell's records into
-// LDS with one wide copy and runs the recorded flushes, so results equal a full traversal.
-constexpr int PC_CELL_MAX = PAIR_CAP + WAVE;  // entries of one cell's records (the LDS list)
-struct PairCache {
-    uint16_t* data;
-    long long region;  // entries per wavefront (multiple of 4)
-    int* head;
-};
-
 template <class T>
 __device__ __forceinline__ T lane_bcast(T v, int i) {
     if constexpr (sizeof(T) == 4) {
@@ -111,16 +96,12 @@ __device__ __forceinline__ void with_groups(int n, Fn&& fn) {
     }
 }
 
-// PCM: pair cache mode of this instance (0 off, 1 record, 2 replay); only functors with
-// kCache use 1 and 2.
 // HASH: the grid is keyed by a SpatialHashingCellList (a work item is a non-empty query
 // bucket, the pieces are the 3^D neighbour cells' buckets) and binned from the current
 // coordinates, so the per-bucket cell and collision flags of the binning hold.  A query
 // bucket that mixes cells is run once per cell, over that cell's queries.
-template <int D, class TC, class TR, class F, int G, bool PER, int PCM, bool HASH = false>
-__global__ __launch_bounds__(WAVE) void k_cells(Geom g, SetView Q, SetView Gs, TR r2, F f, int nblocks,
-                                                PairCache pc) {
-    static_assert(!HASH || PCM == 0, "no pair cache over a hash grid");
+template <int D, class TC, class TR, class F, int G, bool PER, bool HASH = false>
+__global__ __launch_bounds__(WAVE) void k_cells(Geom g, SetView Q, SetView Gs, TR r2, F f, int nblocks) {
     constexpr int R = Rows<D>::R;
     // stencil pieces: rows (two per row with a periodic box), or 3^D buckets
     constexpr int RP = HASH ? (D == 1 ? 3 : (D == 2 ? 9 : 27)) : (PER ? 2 * R : R);
@@ -140,13 +121,9 @@ __global__ __launch_bounds__(WAVE) void k_cells(Geom g, SetView Q, SetView Gs, T
     constexpr int FOFF = kPackF ? 1 : 0;
     constexpr int NFL = NF - FOFF;  // fields kept in their own LDS planes
     __shared__ TR s_f[NFL > 0 ? NFL : 1][(!kLight && NFL > 0) ? CH : 1];
-    // Pair list: candidate slots of the chunk, one byte each when a chunk holds at most 256 and
-    // no pair cache is involved; a replay copies a cell's 16-bit records (up to PC_CELL_MAX
-    // entries) here.
-    using PairT = typename std::conditional<(PCM == 0 && CH <= 256), uint8_t, uint16_t>::type;
-    constexpr int PAIR_WORDS = (PCM == 0 ? (PAIR_CAP + WAVE) * (int)sizeof(PairT) : 2 * PC_CELL_MAX) / 8;
-    __shared__ uint64_t s_pairs64[kLight ? 1 : PAIR_WORDS];
-    PairT* const s_pairs = (PairT*)s_pairs64;
+    // Pair list: candidate slots of the chunk, one byte each when a chunk holds at most 256
+    using PairT = typename std::conditional<(CH <= 256), uint8_t, uint16_t>::type;
+    __shared__ PairT s_pairs[kLight ? 1 : PAIR_CAP + WAVE];
     __shared__ uint16_t s_qstart[LQ + 1];
     // the query batch's coordinates, lane k holding query k's: read with one broadcast LDS load
     // per query in the test loop and per lane in the pair bodies; in Float64 pair functors they
@@ -212,13 +189,6 @@ __global__ __launch_bounds__(WAVE) void k_cells(Geom g, SetView Q, SetView Gs, T
         return d2;
     };
 
-    // Record mode: write position in this wavefront's region, start of the current cell's
-    // records, and whether they all fitted.
-    long long rec_pos = (long long)blockIdx.x * pc.region;
-    const long long rec_end = rec_pos + pc.region;
-    long long cell_base = rec_pos;
-    bool cell_ok = true;
-
     // Runs the pair body over pairs [0, P) of list `prp`, which hold queries i0 .. i1-1
     // (qsp[q - i0] = first pair of query q, qsp[i1 - i0] = P).  The 64 lanes are shared
     // out over the i1 - i0 queries (floor or ceil of 64 / (i1 - i0) each), which take their
@@ -243,28 +213,9 @@ __global__ __launch_bounds__(WAVE) void k_cells(Geom g, SetView Q, SetView Gs, T
         if constexpr (kQstLds) return s_qst[q];
         else return f.query((int64_t)Q.sorted_idx[cur_q0 + q]);
     };
-    auto flush = [&](int i0, int i1, int P, int batch, int chunk, const uint16_t* qsp, const PairT* prp) {
+    auto flush = [&](int i0, int i1, int P, const uint16_t* qsp, const PairT* prp) {
         const int nf = i1 - i0;
         __syncthreads();
-        if constexpr (F::kCache && PCM == 1) {
-            if (cell_ok && P > 0) {
-                const long long size = 5 + nf + P;
-                if (rec_pos + size > rec_end || rec_pos + size - cell_base > PC_CELL_MAX) {
-                    cell_ok = false;
-                } else {
-                    uint16_t* rec = pc.data + rec_pos;
-                    if (lane == 0) {
-                        rec[0] = (uint16_t)batch;
-                        rec[1] = (uint16_t)chunk;
-                        rec[2] = (uint16_t)i0;
-                        rec[3] = (uint16_t)i1;
-                    }
-                    for (int t = lane; t <= nf; t += WAVE) rec[4 + t] = qsp[t];
-                    for (int k = lane; k < P; k += WAVE) rec[5 + nf + k] = prp[k];
-                    rec_pos += size;
-                }
-            }
-        }
         if constexpr (F::kFill) {
             // CSR fill: pair k goes to lane k % 64, so a store instruction writes consecutive
             // slots of one or two rows; each lane's query cursor only moves forward.
@@ -372,9 +323,6 @@ __global__ __launch_bounds__(WAVE) void k_cells(Geom g, SetView Q, SetView Gs, T
     const int wchunk = (n_work + 7) >> 3;
     const int w_end = min(n_work, (xcd + 1) * wchunk);
     for (int w = xcd * wchunk + (int)(blockIdx.x >> 3); w < w_end; w += per_xcd) {
-        cell_base = (rec_pos + 3) & ~3ll;  // 8-byte aligned cell records
-        rec_pos = cell_base;
-        cell_ok = true;
         const int qc = Q.nonempty[w];
         const int qs = Q.start[qc], qe = Q.start[qc + 1];
         // The piece table in scalar registers: element m of piece u sits at sorted position
@@ -665,47 +613,7 @@ __global__ __launch_bounds__(WAVE) void k_cells(Geom g, SetView Q, SetView Gs, T
             }
         };
 
-        int rbase = -1, rsize = 0;
-        if constexpr (F::kCache && PCM == 2) {
-            rbase = pc.head[2 * (int64_t)w];
-            rsize = pc.head[2 * (int64_t)w + 1];
-        }
-        if constexpr (PCM == 2) {
-        if (rbase >= 0) {
-            // replay: copy the cell's records to LDS (8 bytes per lane and step), then run
-            // the recorded flushes batch by batch
-            __syncthreads();
-            const uint64_t* src = (const uint64_t*)pc.data + rbase;
-            for (int k = lane; k < (rsize + 3) / 4; k += WAVE) s_pairs64[k] = src[k];
-            __syncthreads();
-            int pos = 0;
-            for (int q0 = qs, b = 0; q0 < qe; q0 += WAVE, ++b) {
-                const int nq = min(WAVE, qe - q0);
-                TC xq[D];
-                int64_t orig_i;
-                begin_batch(q0, nq, xq, orig_i);
-                int staged = -1;
-                while (pos < rsize && (int)s_pairs[pos] == b) {
-                    const int chunk = s_pairs[pos + 1], i0 = s_pairs[pos + 2], i1 = s_pairs[pos + 3];
-                    const int nf = i1 - i0;
-                    const int P = s_pairs[pos + 4 + nf];
-                    if (chunk != staged) {
-                        const int m0 = chunk * CH;
-                        TC unused[G][D];
-                        stage_lds(m0, min(CH, M - m0), unused);
-                        staged = chunk;
-                    }
-                    flush(i0, i1, P, b, chunk, s_pairs + pos + 4, s_pairs + pos + 5 + nf);
-                    pos += 5 + nf + P;
-                }
-                __syncthreads();
-                if (lane < nq) f.write(orig_i, qstate(lane), query_sum());
-            }
-            continue;
-        }
-        }
-
-        for (int q0 = qs, b = 0; q0 < qe; q0 += WAVE, ++b) {
+        for (int q0 = qs; q0 < qe; q0 += WAVE) {
             const int nq = min(WAVE, qe - q0);
             const bool qact = lane < nq;
             TC xq[D];
@@ -739,7 +647,7 @@ __global__ __launch_bounds__(WAVE) void k_cells(Geom g, SetView Q, SetView Gs, T
                 }
             }
 
-            for (int m0 = 0, chunk = 0; m0 < M; m0 += CH, ++chunk) {
+            for (int m0 = 0; m0 < M; m0 += CH) {
                 const int mc = min(CH, M - m0);
                 const int ng = (mc + WAVE - 1) / WAVE;
                 TC cx[G][D];
@@ -779,7 +687,7 @@ __global__ __launch_bounds__(WAVE) void k_cells(Geom g, SetView Q, SetView Gs, T
                             for (int gi = 0; gi < NG; ++gi)
                                 c += __builtin_popcountll(__builtin_amdgcn_ballot_w64(test(xs, gi)));
                             // lane i holds query i's count (no earlier chunk: nothing to add)
-                            if (chunk != 0) c += __builtin_amdgcn_readlane(mycount, i);
+                            if (m0 != 0) c += __builtin_amdgcn_readlane(mycount, i);
                             mycount = write_lane(mycount, c, i);
                         }
                     });
@@ -791,7 +699,7 @@ __global__ __launch_bounds__(WAVE) void k_cells(Geom g, SetView Q, SetView Gs, T
                         const int nf = i1 - i0;
                         if (lane < nf) s_qstart[lane] = (uint16_t)qfirst;
                         if (lane == 0) s_qstart[nf] = (uint16_t)P;
-                        flush(i0, i1, P, b, chunk, s_qstart, s_pairs);
+                        flush(i0, i1, P, s_qstart, s_pairs);
                     };
                     with_groups<G>(ng, [&](auto ngc) {
                         constexpr int NG = decltype(ngc)::value;
@@ -835,15 +743,6 @@ __global__ __launch_bounds__(WAVE) void k_cells(Geom g, SetView Q, SetView Gs, T
                 if (qact) f.write(orig_i, qstate(lane), query_sum());
             }
 
-        }
-        if constexpr (F::kCache && PCM == 1) {
-            {
-                if (lane == 0) {
-                    pc.head[2 * (int64_t)w] = cell_ok ? (int)(cell_base >> 2) : -1;
-                    pc.head[2 * (int64_t)w + 1] = (int)(rec_pos - cell_base);
-                }
-                if (!cell_ok) rec_pos = cell_base;
-            }
         }
     }
 }

@@ -16,6 +16,7 @@
 #include "pn_sph.h"
 #include "pn_traverse.h"
 #include "pn_cells.h"
+#include "pn_runs.h"
 #include "pn_lists.h"
 
 namespace pn_host {
@@ -142,6 +143,7 @@ struct BinSet {
         v.start = start.as<int32_t>();
         v.nonempty = nonempty.as<int32_t>();
         v.sorted_idx = sorted_idx.as<int32_t>();
+        v.keys = hash_epoch > 0 ? nullptr : slots.as<int32_t>();
         v.coords = coords.p;
         v.cap = cap;
         v.st = status.as<pn::DevStatus>();
@@ -171,13 +173,6 @@ struct pn_grid {
     int chunk = 0;                  // candidate chunk: -1 per functor, 0 small, 1 large
     int algorithm = 0;              // traversal: 0 candidate-major cells, 1 per-query slices
     int canonical_order = 1;        // 1: in-cell order = ascending original index
-    int pair_cache = 0;             // record / replay forward pair lists (pn::PairCache)
-    int64_t pc_per_point = 0;       // cache capacity in entries per point (0: by dimension)
-    uint64_t gen = 0;               // build generation: bumped by every binning or refresh
-    Buf pc_data, pc_head;           // pair cache storage
-    int64_t pc_region = 0;          // entries per wavefront of the recording launch
-    uint64_t pc_gen = ~0ull;        // generation the cache was recorded at
-    int pc_groups = 0;              // candidate groups of the recording kernel
     Buf csr_counts;
     Buf csr_status;
     Scanner csr_scan;
@@ -194,8 +189,6 @@ struct pn_grid {
     ~pn_grid() {
         for (hipEvent_t e : timing_events) (void)hipEventDestroy(e);
         fields.release();
-        pc_data.release();
-        pc_head.release();
         geom_table.release();
         cloud_of.release();
         cell_offs.release();
@@ -321,7 +314,6 @@ unsigned blocks_for(int64_t n, int threads) { return (unsigned)std::max<int64_t>
 // Enqueues the counting-sort binning of the selected points of src into s.
 int enqueue_bin(pn_grid& g, BinSet& s, const void* src, int64_t n_src, int64_t sel_first, int64_t sel_count,
                 const int32_t* sel_list) {
-    ++g.gen;  // recorded pair lists belong to the previous build
     if (!src && sel_count > 0) return fail(PN_ERR_ARGUMENT, "coordinate pointer is NULL");
     if (sel_count < 0 || n_src < 0) return fail(PN_ERR_ARGUMENT, "negative size");
     if (n_src > INT32_MAX - 1 || sel_count > INT32_MAX - 1)
@@ -367,7 +359,8 @@ int enqueue_bin(pn_grid& g, BinSet& s, const void* src, int64_t n_src, int64_t s
                 hipLaunchKernelGGL((pn::k_canon<D, TC>), dim3(blocks_for(sel_count, 256)), dim3(256), 0, g.stream,
                                    s.keys.as<int32_t>(), sel_first, sel_list, (const pn::DevStatus*)st,
                                    s.start.as<int32_t>(), s.perm_tmp.as<int32_t>(), (const TC*)src,
-                                   s.sorted_idx.as<int32_t>(), s.coords.as<TC>(), s.cap, g.canonical_order);
+                                   s.sorted_idx.as<int32_t>(), s.coords.as<TC>(), s.cap, g.canonical_order,
+                                   s.slots.as<int32_t>());
                 PN_CHECK_LAUNCH();
             } else {
                 // mixed-bucket flags of earlier binnings hold earlier epochs; fresh memory (epoch 0)
@@ -535,10 +528,94 @@ int check_queries(pn_grid& g, int queries, const BinSet*& Q) {
     return PN_OK;
 }
 
-// Gathers the functor's per-neighbour fields into sorted order, then launches the
-// wave-per-cell traversal for the query set.
+// Whether the run kernels (pn_runs.h) take a traversal: they need a cell per sorted position
+// (a FullGridCellList), lengths that Float32 holds with room for their squares, and planes that a
+// 32-bit byte offset reaches.  They are faster than the cell kernel (k_cells) over the sizes
+// measured (1M points, F32: count 116 -> 90 us, density 236 -> 152, pressure 238 -> 177, TrixiParticles
+// interact! 623 -> 432, F64 1367 -> 831; 1000 points: count 14.7 -> 10.3, density 24.5 -> 15.7) but
+// for 2D pair functors below about 100,000 points (2000 points: density 7.6 -> 8.9 us) and for
+// counting an undeformed lattice whose search radius is a lattice distance (128^3, r = 3 spacings:
+// 305 -> 400 us, a quarter of the neighbours are ties), so the list builder counts by cells.
+template <class F>
+bool runs_apply(const pn_grid& g) {
+    if ((g.algorithm != 0 && !g.geom.periodic) || g.geom.hash || F::kFill) return false;
+    if (g.grid.cap > (int64_t)1 << 28) return false;
+    if (!(g.radius >= 0x1p-60 && g.radius <= 0x1p60)) return false;
+    if (g.geom.periodic)
+        for (int d = 0; d < g.nd; ++d)
+            if (!(g.geom.box[d] <= 0x1p20 * g.radius)) return false;
+    return true;
+}
+
+// Launch parameters of the run kernels for n query points (known: exactly n, else at most n).
+// Runs of 32 queries do the least work; shorter ones put more wavefronts on a small cloud and end
+// sooner.  Measured at r = 2.4 spacings, F32, us with 8 / 16 / 32: density 15.6 / 18.4 / 22.5 at
+// 15,600 points, 20.5 / 19.3 / 24.1 at 32,768, 30.2 / 24.2 / 23.5 at 64,000, 160 / 105 / 80 at 512,000;
+// count 9.6 / 9.8 / 10.8 at 4096, 14.7 / 12.2 / 12.2 at 32,768, 104 / 62 / 43 at 512,000.  Queries that
+// are sparser than the grid's points have more candidates per run, so more work in each: they count
+// as fewer (100,000 probes among 512,000 bodies: n-body 87 / 68 / 86 us).
+// fresh: the grid was binned from the current coordinates.
+void run_params(const pn_grid& g, int64_t n, bool known, bool light, bool fresh, pn::RunScale& sc, pn::RunSplit& sp) {
+    const pn::Geom& geom = g.geom;
+    const double radius = g.radius;
+    sc = pn::RunScale{};
+    int e;
+    (void)std::frexp(radius, &e);  // radius = m 2^e, m in [1/2, 1)
+    sc.s = (float)std::ldexp(1.0, 1 - e);
+    sc.rt = (float)radius * sc.s;
+    sp.n = known ? (int)n : -1;
+    const int64_t nc = g.grid.n_sel;
+    const double work = n < nc ? (double)n * std::sqrt((double)n / (double)nc) : (double)n;
+    sp.most = light ? (work >= 32768 ? 32 : (work >= 8192 ? 16 : 8)) : (work >= 65536 ? 32 : (work >= 24576 ? 16 : 8));
+    sp.span = pn::RUN_SPAN;
+    sp.magic0 = 0xffffffffu / (unsigned)geom.n[0];
+    sp.magic1 = 0xffffffffu / (unsigned)geom.n[1];
+    if (geom.periodic) {
+        // a run leaves two of the periodic cells out
+        sp.span = std::min(sp.span, geom.per[0] - 2);
+        double len = 0.0;
+        for (int d = 0; d < g.nd; ++d) len += geom.box[d];
+        sc.per_mg = (float)(len * sc.s * sc.rt * 0x1p-19);
+    }
+    // (x - min) / cell size has a relative error below 2 u, so a pair two cells apart is at least
+    // r (1 - 4 u n) away; twice that for d^2, and its own rounding.  Where that bound is useless, or
+    // the cells are those of earlier coordinates, runs are single cells.
+    sp.cell64 = g.tcell == PN_FLOAT64;
+    int64_t n0 = geom.n[0];
+    for (const pn::GeomEntry& e : g.host_table) n0 = std::max<int64_t>(n0, e.n[0]);
+    sc.cell_rel = (double)(n0 + 1) * (sp.cell64 ? 0x1p-49 : 0x1p-20) + (g.tr == PN_FLOAT64 ? 0x1p-48 : 0x1p-20);
+    if (sc.cell_rel > 0x1p-6 || !fresh) sp.span = 1;
+}
+
 template <int D, class TC, class TR, class F>
-int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* src) {
+int launch_runs(pn_grid& g, const BinSet* Q, const F& f) {
+    const int64_t n = Q->stats_known ? Q->stats.n_binned : Q->n_sel;
+    if (n == 0) return PN_OK;
+    const TR r = (TR)g.radius, r2 = r * r;
+    pn::RunScale sc;
+    pn::RunSplit sp;
+    run_params(g, n, Q->stats_known, F::kLight, g.grid.fresh, sc, sp);
+    const int nblocks = (int)std::min<int64_t>(round_up8((n + sp.most - 1) / sp.most), g.persist_blocks);
+    LaunchTimer timer(g);  // brackets the one traversal kernel launched below
+    auto launch = [&](auto perc) {
+        constexpr bool PER = decltype(perc)::value;
+        if constexpr (F::kLight)
+            hipLaunchKernelGGL((pn::k_runs_count<D, TC, TR, PER>), dim3(nblocks), dim3(pn::WAVE), 0, g.stream, g.geom,
+                               Q->view(), g.grid.view(), r2, f, nblocks, sc, sp);
+        else
+            hipLaunchKernelGGL((pn::k_runs<D, TC, TR, F, PER>), dim3(nblocks), dim3(pn::WAVE), 0, g.stream, g.geom,
+                               Q->view(), g.grid.view(), r2, f, nblocks, sc, sp);
+    };
+    if (g.geom.periodic) launch(std::true_type{});
+    else launch(std::false_type{});
+    PN_CHECK_LAUNCH();
+    return PN_OK;
+}
+
+// Gathers the functor's per-neighbour fields into sorted order, then launches the
+// traversal for the query set.
+template <int D, class TC, class TR, class F>
+int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* src, bool allow_runs = true) {
     if (Q->n_sel == 0) return PN_OK;
     if constexpr (F::kFields > 0) {
         const BinSet& G = g.grid;
@@ -553,6 +630,9 @@ int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* 
         }
         f.fsorted = g.fields.p;
         f.fstride = stride;
+    }
+    if constexpr (!F::kFill) {
+        if (allow_runs && runs_apply<F>(g)) return launch_runs<D, TC, TR, F>(g, Q, f);
     }
     // Upper bound on non-empty query cells; the kernel reads the exact count on device.
     int64_t nwork = std::min<int64_t>(g.geom.ncells, Q->n_sel);
@@ -590,8 +670,8 @@ int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* 
         auto launch_hc = [&](auto gc, auto perc) {
             constexpr int GG = decltype(gc)::value;
             constexpr bool PER = decltype(perc)::value;
-            hipLaunchKernelGGL((pn::k_cells<D, TC, TR, F, GG, PER, 0, true>), dim3(nblocks), dim3(pn::WAVE), 0,
-                               g.stream, g.geom, Q->view(), g.grid.view(), r2, f, nblocks, pn::PairCache{});
+            hipLaunchKernelGGL((pn::k_cells<D, TC, TR, F, GG, PER, true>), dim3(nblocks), dim3(pn::WAVE), 0, g.stream,
+                               g.geom, Q->view(), g.grid.view(), r2, f, nblocks);
         };
         using Large = pn::IntC<pn::CellGroups<TC, F>::large>;
         using Small = pn::IntC<pn::CellGroups<TC, F>::small>;
@@ -605,64 +685,14 @@ int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* 
         PN_CHECK_LAUNCH();
         return PN_OK;
     }
-    if (g.algorithm == 0 || g.geom.periodic) {  // only the cell kernel handles periodic boxes
-        pn::PairCache pc{};
-        int pcm = 0;  // pair cache mode of the launch
-        auto launch = [&](auto gc, auto perc) {
-            constexpr int GG = decltype(gc)::value;
-            constexpr bool PER = decltype(perc)::value;
-            if constexpr (F::kCache && !PER) {
-                if (pcm == 1) {
-                    hipLaunchKernelGGL((pn::k_cells<D, TC, TR, F, GG, PER, 1>), dim3(nblocks), dim3(pn::WAVE), 0,
-                                       g.stream, g.geom, Q->view(), g.grid.view(), r2, f, nblocks, pc);
-                    return;
-                }
-                if (pcm == 2) {
-                    hipLaunchKernelGGL((pn::k_cells<D, TC, TR, F, GG, PER, 2>), dim3(nblocks), dim3(pn::WAVE), 0,
-                                       g.stream, g.geom, Q->view(), g.grid.view(), r2, f, nblocks, pc);
-                    return;
-                }
-            }
-            hipLaunchKernelGGL((pn::k_cells<D, TC, TR, F, GG, PER, 0>), dim3(nblocks), dim3(pn::WAVE), 0, g.stream,
-                               g.geom, Q->view(), g.grid.view(), r2, f, nblocks, pc);
-        };
-        using Large = pn::IntC<pn::CellGroups<TC, F>::large>;
-        using Small = pn::IntC<pn::CellGroups<TC, F>::small>;
-        if constexpr (F::kCache) {
-            if (g.pair_cache && Q == &g.grid && !g.geom.periodic) {
-                const int groups = g.chunk != 0 ? Large::value : Small::value;
-                int rc = PN_OK;
-                // per wavefront: its share of about `per_point` entries per point, at least one
-                // cell's records
-                const int64_t per_point = g.pc_per_point > 0 ? g.pc_per_point : (D == 3 ? 108 : (D == 2 ? 36 : 12));
-                int64_t region = (Q->n_sel * per_point + nblocks - 1) / nblocks;
-                if (g.pc_per_point == 0) region = std::max<int64_t>(region, pn::PC_CELL_MAX + 8);
-                region = (region + 3) & ~int64_t(3);
-                const int64_t cap = region * nblocks;
-                if (cap / 4 > INT32_MAX) return fail(PN_ERR_UNSUPPORTED, "pair cache larger than 2^33 entries");
-                if ((rc = g.pc_head.ensure((size_t)nwork * 8, g.stream)) ||
-                    (rc = g.pc_data.ensure((size_t)cap * 2, g.stream)))
-                    return rc;
-                pc.data = g.pc_data.as<uint16_t>();
-                pc.region = (long long)region;
-                pc.head = g.pc_head.as<int>();
-                if (g.pc_gen == g.gen && g.pc_groups == groups && g.pc_region == region) {
-                    pcm = 2;
-                } else {
-                    pcm = 1;
-                    g.pc_gen = g.gen;
-                    g.pc_groups = groups;
-                    g.pc_region = region;
-                }
-            }
-        }
-        if (g.geom.periodic) {
-            if (g.chunk != 0) launch(Large{}, std::true_type{});
-            else launch(Small{}, std::true_type{});
-        } else {
-            if (g.chunk != 0) launch(Large{}, std::false_type{});
-            else launch(Small{}, std::false_type{});
-        }
+    if (g.algorithm == 0 || g.geom.periodic) {  // k_traverse does not handle periodic boxes
+        constexpr int GG = pn::CellGroups<TC, F>::small;
+        if (g.geom.periodic)
+            hipLaunchKernelGGL((pn::k_cells<D, TC, TR, F, GG, true>), dim3(nblocks), dim3(pn::WAVE), 0, g.stream,
+                               g.geom, Q->view(), g.grid.view(), r2, f, nblocks);
+        else
+            hipLaunchKernelGGL((pn::k_cells<D, TC, TR, F, GG, false>), dim3(nblocks), dim3(pn::WAVE), 0, g.stream,
+                               g.geom, Q->view(), g.grid.view(), r2, f, nblocks);
         PN_CHECK_LAUNCH();
         return PN_OK;
     }
@@ -678,7 +708,7 @@ int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* 
 }
 
 template <class F>
-int launch_traverse(pn_grid& g, int queries, const F& f) {
+int launch_traverse(pn_grid& g, int queries, const F& f, bool allow_runs = true) {
     const BinSet* Q;
     int rc = check_queries(g, queries, Q);
     if (rc) return rc;
@@ -686,7 +716,7 @@ int launch_traverse(pn_grid& g, int queries, const F& f) {
         constexpr int D = decltype(dc)::value;
         using TC = decltype(tcv);
         using TR = decltype(trv);
-        return launch_traverse_t<D, TC, TR, F>(g, Q, f, (const pn::FieldSrc<TR>*)nullptr);
+        return launch_traverse_t<D, TC, TR, F>(g, Q, f, (const pn::FieldSrc<TR>*)nullptr, allow_runs);
     });
 }
 
