@@ -309,6 +309,22 @@ int pn_list_sph_density(const int32_t* row_ptr, const int32_t* col_idx, int64_t 
                         int64_t sel_count, const int32_t* sel_list, void* rho, int accumulate,
                         void* stream);
 
+/* pn_list_sph_density (box_size NULL) or pn_list_sph_density_periodic with one floating type and
+ * a workspace of pn_list_pack_bytes(dtype, n_y) bytes of 16-byte aligned device memory, n_y > 0
+ * the points of y: the call first packs each point's coordinates and mass into one record
+ * there and gathers those (same results bit for bit, fewer loads).  Pays from about 12 million
+ * entries in the selected rows.  Enqueue only. */
+int pn_list_sph_density_packed(const int32_t* row_ptr, const int32_t* col_idx, int64_t n_rows,
+                               int stored_base, int ndims, int dtype, int kernel, double h,
+                               const void* x, const void* y, int64_t n_y, const void* mass,
+                               int64_t sel_first, int64_t sel_count, const int32_t* sel_list, void* rho,
+                               int accumulate, double search_radius, const double* box_size,
+                               void* workspace, void* stream);
+
+/* Size in bytes of n records of the packed list calls: four values each (-1 for an unsupported
+ * dtype).  No counterpart in the reference (an implementation buffer). */
+int64_t pn_list_pack_bytes(int dtype, int64_t n);
+
 /* CSR lists (pn_csr_fill) -> the reference's DynamicVectorOfVectors{Int32} backend
  * (src/vector_of_vectors.jl:3-31; PrecomputedNeighborhoodSearch's `backend` and
  * `transpose_backend`, src/nhs_precomputed.jl:40-66).  lengths[i] = length of row i.  Entry k of
@@ -336,6 +352,18 @@ int pn_list_tlsph_deformation_grad(const int32_t* row_ptr, const int32_t* col_id
                                    const void* X, const void* x, const void* volume, const void* L,
                                    int invert, int64_t sel_first, int64_t sel_count,
                                    const int32_t* sel_list, void* out, void* stream);
+
+/* pn_list_tlsph_deformation_grad with a workspace of pn_list_pack_bytes(dtype, 2 * n_rows) bytes
+ * of 16-byte aligned device memory; the lists are X's own (n_rows = N).  The call first packs
+ * X, volume and x into records there and gathers those (same results bit for bit, fewer
+ * loads).  dtype must be PN_FLOAT32.  Pays from about 12 million entries in the selected rows.
+ * Enqueue only. */
+int pn_list_tlsph_deformation_grad_packed(const int32_t* row_ptr, const int32_t* col_idx, int64_t n_rows,
+                                          int stored_base, int ndims, int dtype, int kernel, double h,
+                                          const void* X, const void* x, const void* volume, const void* L,
+                                          int invert, int64_t sel_first, int64_t sel_count,
+                                          const int32_t* sel_list, void* out, void* workspace,
+                                          void* stream);
 
 /* TLSPH interaction forces over the same stored lists (TrixiParticles 0.5
  * interact_structure_structure!, the loop the reference times in benchmark_tlsph,

@@ -407,7 +407,7 @@ static int list_sph_density(const int32_t* row_ptr, const int32_t* col_idx, int6
                             int ndims, int coord_dtype, int radius_dtype, int kernel, double h, const void* x,
                             const void* y, const void* mass, int64_t sel_first, int64_t sel_count,
                             const int32_t* sel_list, void* rho, int accumulate, void* stream, double search_radius,
-                            const double* box_size) {
+                            const double* box_size, int64_t n_y = 0, void* workspace = nullptr) {
     if (!row_ptr || !x || !y || !mass || !rho) return fail(PN_ERR_ARGUMENT, "NULL pointer");
     if (ndims != 2 && ndims != 3) return fail(PN_ERR_UNSUPPORTED, "the SPH kernels are defined for 2D and 3D");
     if (kernel != pn::KERNEL_CUBIC_SPLINE && kernel != pn::KERNEL_WENDLAND_C2)
@@ -431,13 +431,33 @@ static int list_sph_density(const int32_t* row_ptr, const int32_t* col_idx, int6
         const int nblocks = (int)round_up8((sel_count + rows - 1) / rows);
         auto kern = pn::SmoothingKernel<TR, D>::make(kernel, h);
         pn::ListPeriodic<TR> per{};
-        per.on = box_size ? 1 : 0;
         const TR r = (TR)search_radius;
         per.r2 = r * r;
         for (int d = 0; d < 3; ++d) per.box[d] = (box_size && d < D) ? (TR)box_size[d] : (TR)1;
-        hipLaunchKernelGGL((pn::k_list_density<D, TC, TR, pn::SmoothingKernel<TR, D>>), dim3(nblocks), dim3(256),
-                           0, (hipStream_t)stream, row_ptr, col_idx, stored_base, sel_first, sel_list, sel_count,
-                           (const TC*)x, (const TC*)y, (const TR*)mass, kern, (TR*)rho, accumulate, nblocks, per);
+        using K = pn::SmoothingKernel<TR, D>;
+        auto go = [&](auto kernel_fn, const pn::ListRec<TR>* rec) {
+            hipLaunchKernelGGL(kernel_fn, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, row_ptr, col_idx,
+                               stored_base, sel_first, sel_list, sel_count, (const TC*)x, (const TC*)y,
+                               (const TR*)mass, rec, kern, (TR*)rho, accumulate, nblocks, per);
+        };
+        if constexpr (std::is_same<TC, TR>::value) {
+            if (workspace) {
+                auto* rec = (pn::ListRec<TR>*)workspace;
+                hipLaunchKernelGGL((pn::k_list_pack<D, TR>), dim3(blocks_for(n_y, 256)), dim3(256), 0,
+                                   (hipStream_t)stream, (const TR*)y, (const TR*)mass, (const TR*)nullptr, n_y, rec);
+                PN_CHECK_LAUNCH();
+                if (box_size)
+                    go(pn::k_list_density<D, TC, TR, K, true, true>, rec);
+                else
+                    go(pn::k_list_density<D, TC, TR, K, true, false>, rec);
+                PN_CHECK_LAUNCH();
+                return PN_OK;
+            }
+        }
+        if (box_size)
+            go(pn::k_list_density<D, TC, TR, K, false, true>, nullptr);
+        else
+            go(pn::k_list_density<D, TC, TR, K, false, false>, nullptr);
         PN_CHECK_LAUNCH();
         return PN_OK;
     });
@@ -461,10 +481,11 @@ int pn_csr_to_dvov(const int32_t* row_ptr, const int32_t* col_idx, int64_t n_row
     return PN_OK;
 }
 
-int pn_list_tlsph_deformation_grad(const int32_t* row_ptr, const int32_t* col_idx, int64_t n_rows, int stored_base,
-                                   int ndims, int dtype, int kernel, double h, const void* X, const void* x,
-                                   const void* volume, const void* L, int invert, int64_t sel_first,
-                                   int64_t sel_count, const int32_t* sel_list, void* out, void* stream) {
+static int list_tlsph_deformation_grad(const int32_t* row_ptr, const int32_t* col_idx, int64_t n_rows,
+                                       int stored_base, int ndims, int dtype, int kernel, double h, const void* X,
+                                       const void* x, const void* volume, const void* L, int invert,
+                                       int64_t sel_first, int64_t sel_count, const int32_t* sel_list, void* out,
+                                       void* workspace, void* stream) {
     if (!row_ptr || !X || !x || !volume || !out) return fail(PN_ERR_ARGUMENT, "NULL pointer");
     if (ndims != 2 && ndims != 3) return fail(PN_ERR_UNSUPPORTED, "the TLSPH kernels are defined for 2D and 3D");
     if (kernel != pn::KERNEL_CUBIC_SPLINE && kernel != pn::KERNEL_WENDLAND_C2)
@@ -472,6 +493,9 @@ int pn_list_tlsph_deformation_grad(const int32_t* row_ptr, const int32_t* col_id
     if (!(h > 0.0)) return fail(PN_ERR_ARGUMENT, "smoothing length must be positive");
     if (dtype != PN_FLOAT32 && dtype != PN_FLOAT64) return fail(PN_ERR_ARGUMENT, "dtype must be PN_FLOAT32 or PN_FLOAT64");
     if (invert && L) return fail(PN_ERR_ARGUMENT, "invert needs L == NULL");
+    if (((uintptr_t)workspace & 15u) != 0) return fail(PN_ERR_ARGUMENT, "workspace must be 16-byte aligned");
+    if (workspace && dtype != PN_FLOAT32)
+        return fail(PN_ERR_UNSUPPORTED, "the packed deformation gradient is defined for PN_FLOAT32");
     if (!sel_list && (sel_first < 0 || sel_first + sel_count > n_rows))
         return fail(PN_ERR_ARGUMENT, "selection range out of bounds of the neighbor lists");
     if (sel_count <= 0) return PN_OK;
@@ -481,15 +505,52 @@ int pn_list_tlsph_deformation_grad(const int32_t* row_ptr, const int32_t* col_id
         constexpr int rows = pn::ListShape<T, true>::rows;
         const int nblocks = (int)round_up8((sel_count + rows - 1) / rows);
         auto kern = pn::SmoothingKernel<T, D>::make(kernel, h);
-        hipLaunchKernelGGL((pn::k_list_tlsph_grad<D, T, pn::SmoothingKernel<T, D>>), dim3(nblocks), dim3(256), 0,
-                           (hipStream_t)stream, row_ptr, col_idx, stored_base, sel_first, sel_list, sel_count,
-                           (const T*)X, (const T*)x, (const T*)volume, kern, (const T*)L, invert ? 1 : 0, (T*)out,
-                           nblocks);
+        using K = pn::SmoothingKernel<T, D>;
+        auto go = [&](auto kernel_fn, const pn::ListRec<T>* rec) {
+            hipLaunchKernelGGL(kernel_fn, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, row_ptr, col_idx,
+                               stored_base, sel_first, sel_list, sel_count, (const T*)X, (const T*)x,
+                               (const T*)volume, rec, kern, (const T*)L, invert ? 1 : 0, (T*)out, nblocks);
+        };
+        if constexpr (sizeof(T) == 4) {
+            if (workspace) {
+                auto* rec = (pn::ListRec<T>*)workspace;
+                hipLaunchKernelGGL((pn::k_list_pack<D, T>), dim3(blocks_for(n_rows, 256)), dim3(256), 0,
+                                   (hipStream_t)stream, (const T*)X, (const T*)volume, (const T*)x, n_rows, rec);
+                PN_CHECK_LAUNCH();
+                go(pn::k_list_tlsph_grad<D, T, K, true>, rec);
+                PN_CHECK_LAUNCH();
+                return PN_OK;
+            }
+        }
+        go(pn::k_list_tlsph_grad<D, T, K, false>, nullptr);
         PN_CHECK_LAUNCH();
         return PN_OK;
     };
     if (ndims == 2) return dtype == PN_FLOAT32 ? run(pn::IntC<2>{}, 0.0f) : run(pn::IntC<2>{}, 0.0);
     return dtype == PN_FLOAT32 ? run(pn::IntC<3>{}, 0.0f) : run(pn::IntC<3>{}, 0.0);
+}
+
+int pn_list_tlsph_deformation_grad(const int32_t* row_ptr, const int32_t* col_idx, int64_t n_rows, int stored_base,
+                                   int ndims, int dtype, int kernel, double h, const void* X, const void* x,
+                                   const void* volume, const void* L, int invert, int64_t sel_first,
+                                   int64_t sel_count, const int32_t* sel_list, void* out, void* stream) {
+    return list_tlsph_deformation_grad(row_ptr, col_idx, n_rows, stored_base, ndims, dtype, kernel, h, X, x, volume,
+                                       L, invert, sel_first, sel_count, sel_list, out, nullptr, stream);
+}
+
+int pn_list_tlsph_deformation_grad_packed(const int32_t* row_ptr, const int32_t* col_idx, int64_t n_rows,
+                                          int stored_base, int ndims, int dtype, int kernel, double h,
+                                          const void* X, const void* x, const void* volume, const void* L,
+                                          int invert, int64_t sel_first, int64_t sel_count, const int32_t* sel_list,
+                                          void* out, void* workspace, void* stream) {
+    if (!workspace) return fail(PN_ERR_ARGUMENT, "NULL pointer");
+    return list_tlsph_deformation_grad(row_ptr, col_idx, n_rows, stored_base, ndims, dtype, kernel, h, X, x, volume,
+                                       L, invert, sel_first, sel_count, sel_list, out, workspace, stream);
+}
+
+int64_t pn_list_pack_bytes(int dtype, int64_t n) {
+    if ((dtype != PN_FLOAT32 && dtype != PN_FLOAT64) || n < 0) return -1;
+    return n * (dtype == PN_FLOAT32 ? (int64_t)sizeof(pn::ListRec<float>) : (int64_t)sizeof(pn::ListRec<double>));
 }
 
 int pn_list_tlsph_interaction(const int32_t* row_ptr, const int32_t* col_idx, int64_t n_rows, int stored_base,
@@ -519,14 +580,17 @@ int pn_list_tlsph_interaction(const int32_t* row_ptr, const int32_t* col_idx, in
         auto kern = K::make(kernel, h);
         const T hae = (T)(0.5 * penalty_alpha * young_modulus);
         if (pen && workspace) {
+            constexpr int threads = pn::ListShape<T, true>::rec_threads;
+            constexpr int rec_rows = threads / pn::ListShape<T, true>::lanes;
+            const int rec_blocks = (int)round_up8((sel_count + rec_rows - 1) / rec_rows);
             uint4* rec = (uint4*)workspace;
             hipLaunchKernelGGL((pn::k_tlsph_pack<D, T>), dim3(blocks_for(n_rows, 256)), dim3(256), 0,
                                (hipStream_t)stream, (const T*)X, (const T*)x, (const T*)mass, (const T*)rho,
                                (const T*)pk1_rho2, (const T*)F, n_rows, rec);
             PN_CHECK_LAUNCH();
-            hipLaunchKernelGGL((pn::k_list_tlsph_force_rec<D, T, K>), dim3(nblocks), dim3(256), 0, (hipStream_t)stream,
-                               row_ptr, col_idx, stored_base, sel_first, sel_list, sel_count, rec, (const T*)rho, hae,
-                               kern, (T*)dv, accumulate ? 1 : 0, nblocks);
+            hipLaunchKernelGGL((pn::k_list_tlsph_force_rec<D, T, K>), dim3(rec_blocks), dim3(threads), 0,
+                               (hipStream_t)stream, row_ptr, col_idx, stored_base, sel_first, sel_list, sel_count, rec,
+                               (const T*)rho, hae, kern, (T*)dv, accumulate ? 1 : 0, rec_blocks);
         } else if (pen)
             hipLaunchKernelGGL((pn::k_list_tlsph_force<D, T, K, true>), dim3(nblocks), dim3(256), 0,
                                (hipStream_t)stream, row_ptr, col_idx, stored_base, sel_first, sel_list, sel_count,
@@ -589,6 +653,19 @@ int pn_list_sph_density_periodic(const int32_t* row_ptr, const int32_t* col_idx,
     if (!box_size) return fail(PN_ERR_ARGUMENT, "NULL pointer");
     return list_sph_density(row_ptr, col_idx, n_rows, stored_base, ndims, coord_dtype, radius_dtype, kernel, h, x, y,
                             mass, sel_first, sel_count, sel_list, rho, accumulate, stream, search_radius, box_size);
+}
+
+int pn_list_sph_density_packed(const int32_t* row_ptr, const int32_t* col_idx, int64_t n_rows, int stored_base,
+                               int ndims, int dtype, int kernel, double h, const void* x, const void* y,
+                               int64_t n_y, const void* mass, int64_t sel_first, int64_t sel_count,
+                               const int32_t* sel_list, void* rho, int accumulate, double search_radius,
+                               const double* box_size, void* workspace, void* stream) {
+    if (!workspace) return fail(PN_ERR_ARGUMENT, "NULL pointer");
+    if (((uintptr_t)workspace & 15u) != 0) return fail(PN_ERR_ARGUMENT, "workspace must be 16-byte aligned");
+    if (n_y <= 0) return fail(PN_ERR_ARGUMENT, "n_y must be positive");
+    return list_sph_density(row_ptr, col_idx, n_rows, stored_base, ndims, dtype, dtype, kernel, h, x, y, mass,
+                            sel_first, sel_count, sel_list, rho, accumulate, stream, search_radius, box_size, n_y,
+                            workspace);
 }
 
 }  // extern "C"

@@ -244,7 +244,6 @@ static __global__ __launch_bounds__(256) void k_csr_to_dvov_rows(const int32_t* 
 // (src/neighborhood_search.jl:428-436) applies when on != 0.
 template <class TR>
 struct ListPeriodic {
-    int on;
     TR r2;
     TR box[3];
 };
@@ -256,7 +255,44 @@ struct ListPeriodic {
 // coordinates and masses, so a row's loads are in flight together; the lanes' partial sums
 // are combined in a fixed butterfly order.  x and y are D x N coordinate matrices (original
 // order), mass per y point, rho per x point.
-constexpr int LIST_UNROLL = 4;  // measured best of 1, 2, 4, 8 for the density sum
+//
+// What bounds it is the gathers: the cache lines that each load instruction of a wave touches.
+// Unpacked, a neighbour's coordinates and mass are D + 1 loads.  PACK reads {y, m} records of
+// four values that k_list_pack wrote in the same call, one 16-byte load a neighbour (Float64
+// two).  With 113 neighbours a point, pack included, lattice order / shuffled points:
+// 128^3 Float32 546 -> 388 / 6841 -> 3629 us, Float64 700 -> 552 / 7584 -> 3980 us; 32^3 10 -> 10
+// and 25 -> 17 us.  The lanes add the same terms in the same order: the same bits.
+constexpr int LIST_UNROLL = 4;         // measured best of 1, 2, 4, 8 for the density sum
+constexpr int LIST_UNROLL_PACKED = 2;  // 1: 524 us, 2: 388, 3: 400, 4: 414, 8: 436
+
+// Records of the packed list kernels: four values a point, {p (D), m, 0...}, so that one point
+// is one 16-byte load in Float32 and two in Float64.
+template <class T>
+using ListRec = T __attribute__((ext_vector_type(4)));
+
+template <int D, class T>
+__device__ __forceinline__ ListRec<T> list_rec(const T* __restrict__ p, T m, int64_t i) {
+    ListRec<T> r = {(T)0, (T)0, (T)0, (T)0};
+#pragma unroll
+    for (int d = 0; d < D; ++d) r[d] = p[(int64_t)D * i + d];
+    r[3] = m;
+    return r;
+}
+
+// rec[i] = {p_i, w_i}; with q (the current coordinates of the deformation gradient) the pair
+// rec[2 i] = {p_i, w_i}, rec[2 i + 1] = {q_i, 0}.
+template <int D, class T>
+__global__ __launch_bounds__(256) void k_list_pack(const T* __restrict__ p, const T* __restrict__ w,
+                                                   const T* __restrict__ q, int64_t n, ListRec<T>* __restrict__ rec) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    if (q) {
+        rec[2 * i] = list_rec<D, T>(p, w[i], i);
+        rec[2 * i + 1] = list_rec<D, T>(q, (T)0, i);
+    } else {
+        rec[i] = list_rec<D, T>(p, w[i], i);
+    }
+}
 
 // Lanes per row of the list kernels (a power of two dividing 64) and rows per 256-thread
 // block.  Fewer lanes per row put more rows in flight and shorten the closing butterfly: 8
@@ -268,18 +304,25 @@ template <class T, bool TLSPH>
 struct ListShape {
     static constexpr int lanes = (TLSPH && sizeof(T) == 4) ? 16 : 8;
     static constexpr int rows = 256 / lanes;
+    // Threads of a workgroup of the packed interaction kernel, whose rows' records then share
+    // the compute unit's cache over more neighbouring rows: Float32 512 (821 us on the 101^3
+    // lists, 859 with 256); Float64 256 (1643 us; 512 and more did not gain, 1024 2.4 ms).
+    static constexpr int rec_threads = sizeof(T) == 4 ? 512 : 256;
 };
 
-template <int D, class TC, class TR, class K>
+template <int D, class TC, class TR, class K, bool PACK, bool PER>
 __global__ __launch_bounds__(256) void k_list_density(const int32_t* __restrict__ row_ptr,
                                                       const int32_t* __restrict__ col, int stored_base,
                                                       int64_t sel_first, const int32_t* __restrict__ sel_list,
                                                       int64_t n_sel, const TC* __restrict__ x,
                                                       const TC* __restrict__ y, const TR* __restrict__ mass,
-                                                      K kern, TR* __restrict__ rho, int accumulate, int nblocks,
+                                                      const ListRec<TR>* __restrict__ rec, K kern,
+                                                      TR* __restrict__ rho, int accumulate, int nblocks,
                                                       ListPeriodic<TR> per) {
+    static_assert(!PACK || std::is_same<TC, TR>::value, "records hold one type");
     constexpr int LIST_LANES = ListShape<TR, false>::lanes;
     constexpr int LIST_ROWS_PER_BLOCK = ListShape<TR, false>::rows;
+    constexpr int U = PACK ? LIST_UNROLL_PACKED : LIST_UNROLL;
     const int sub = threadIdx.x & (LIST_LANES - 1);
     const int64_t a = (int64_t)xcd_remap(blockIdx.x, nblocks) * LIST_ROWS_PER_BLOCK + (threadIdx.x / LIST_LANES);
     if (a >= n_sel) return;  // a row's lanes leave together
@@ -289,24 +332,31 @@ __global__ __launch_bounds__(256) void k_list_density(const int32_t* __restrict_
 #pragma unroll
     for (int d = 0; d < D; ++d) xi[d] = x[(int64_t)D * i + d];
     TR s = (TR)0;
-    for (int k0 = b + sub; k0 < e; k0 += LIST_LANES * LIST_UNROLL) {
-        int64_t j[LIST_UNROLL];
+    for (int k0 = b + sub; k0 < e; k0 += LIST_LANES * U) {
+        int j[U];
 #pragma unroll
-        for (int u = 0; u < LIST_UNROLL; ++u) {
+        for (int u = 0; u < U; ++u) {
             const int k = k0 + LIST_LANES * u;
-            j[u] = k < e ? (int64_t)col[k] - stored_base : -1;
+            j[u] = k < e ? col[k] - stored_base : -1;
         }
-        TC yv[LIST_UNROLL][D];
-        TR mv[LIST_UNROLL];
+        TC yv[U][D];
+        TR mv[U];
 #pragma unroll
-        for (int u = 0; u < LIST_UNROLL; ++u) {
+        for (int u = 0; u < U; ++u) {
             const int64_t jj = j[u] >= 0 ? j[u] : 0;
+            if constexpr (PACK) {
+                const ListRec<TR> r = rec[jj];
 #pragma unroll
-            for (int d = 0; d < D; ++d) yv[u][d] = y[(int64_t)D * jj + d];
-            mv[u] = mass[jj];
+                for (int d = 0; d < D; ++d) yv[u][d] = r[d];
+                mv[u] = r[3];
+            } else {
+#pragma unroll
+                for (int d = 0; d < D; ++d) yv[u][d] = y[(int64_t)D * jj + d];
+                mv[u] = mass[jj];
+            }
         }
 #pragma unroll
-        for (int u = 0; u < LIST_UNROLL; ++u) {
+        for (int u = 0; u < U; ++u) {
             TR pd[D];
 #pragma unroll
             for (int d = 0; d < D; ++d) pd[d] = (TR)(xi[d] - yv[u][d]);
@@ -316,7 +366,7 @@ __global__ __launch_bounds__(256) void k_list_density(const int32_t* __restrict_
                 const TR p2 = pd[d] * pd[d];
                 d2 = d2 + p2;
             }
-            if (per.on && d2 > per.r2) {
+            if (PER && d2 > per.r2) {
 #pragma unroll
                 for (int d = 0; d < D; ++d) {
                     const TR kk = rint(pd[d] / per.box[d]);
@@ -348,13 +398,20 @@ __global__ __launch_bounds__(256) void k_list_density(const int32_t* __restrict_
 // With x = X this is the (symmetric) kernel-gradient correction matrix M_a, and L = M^-1
 // (invert) makes G reproduce affine maps exactly.  ListShape lanes
 // per row as in k_list_density; each lane keeps its D x D partial sum, the butterfly over the
-// lanes has a fixed order.  X, x: D x N; out and L: D x D per point, column-major.
-template <int D, class T, class K>
+// lanes has a fixed order.  X, x: D x N; out and L: D x D per point, column-major.  PACK
+// gathers the records rec[2 j] = {X, V}, rec[2 j + 1] = {x, 0} (as in k_list_density, the lines
+// that the gathers touch bound it; Float32 alone): with 113 neighbours a point, pack included,
+// lattice order / shuffled, 128^3 668 -> 550 / 6754 -> 3872 us, 64 x 64 x 32 45 -> 38 / 136 -> 95.
+// Two arrays instead of the pair measured 10 us faster in order and no faster shuffled.  A
+// Float64 record is 64 bytes, which lattice order loses on (100^3 418 -> 513 us).
+template <int D, class T, class K, bool PACK>
 __global__ __launch_bounds__(256) void k_list_tlsph_grad(const int32_t* __restrict__ row_ptr,
                                                          const int32_t* __restrict__ col, int stored_base,
                                                          int64_t sel_first, const int32_t* __restrict__ sel_list,
                                                          int64_t n_sel, const T* __restrict__ X, const T* __restrict__ x,
-                                                         const T* __restrict__ vol, K kern, const T* __restrict__ L,
+                                                         const T* __restrict__ vol,
+                                                         const ListRec<T>* __restrict__ rec, K kern,
+                                                         const T* __restrict__ L,
                                                          int invert, T* __restrict__ out, int nblocks) {
     constexpr int LIST_LANES = ListShape<T, true>::lanes;
     constexpr int LIST_ROWS_PER_BLOCK = ListShape<T, true>::rows;
@@ -376,24 +433,36 @@ __global__ __launch_bounds__(256) void k_list_tlsph_grad(const int32_t* __restri
 #pragma unroll
         for (int c = 0; c < D; ++c) g[r][c] = (T)0;
     }
-    constexpr int UG = 2;  // gathers in flight per lane: 2 measured 1.7x faster than 8 (occupancy)
+    // gathers in flight per lane: 2 measured 1.7x faster than 8 (occupancy); packed 1, 2, 3 and
+    // 4 take 647, 550, 584 and 561 us (128^3)
+    constexpr int UG = 2;
     for (int k0 = b + sub; k0 < e; k0 += LIST_LANES * UG) {
-        int64_t j[UG];
+        int j[UG];
 #pragma unroll
         for (int u = 0; u < UG; ++u) {
             const int k = k0 + LIST_LANES * u;
-            j[u] = k < e ? (int64_t)col[k] - stored_base : -1;
+            j[u] = k < e ? col[k] - stored_base : -1;
         }
         T Xj[UG][D], xj[UG][D], vj[UG];
 #pragma unroll
         for (int u = 0; u < UG; ++u) {
             const int64_t jj = j[u] >= 0 ? j[u] : 0;
+            if constexpr (PACK) {
+                const ListRec<T> r = rec[2 * jj], q = rec[2 * jj + 1];
 #pragma unroll
-            for (int d = 0; d < D; ++d) {
-                Xj[u][d] = X[(int64_t)D * jj + d];
-                xj[u][d] = x[(int64_t)D * jj + d];
+                for (int d = 0; d < D; ++d) {
+                    Xj[u][d] = r[d];
+                    xj[u][d] = q[d];
+                }
+                vj[u] = r[3];
+            } else {
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    Xj[u][d] = X[(int64_t)D * jj + d];
+                    xj[u][d] = x[(int64_t)D * jj + d];
+                }
+                vj[u] = vol[jj];
             }
-            vj[u] = vol[jj];
         }
 #pragma unroll
         for (int u = 0; u < UG; ++u) {
@@ -661,9 +730,15 @@ __device__ __forceinline__ void load_rec(const uint4* __restrict__ rec, int64_t 
 }
 
 // k_list_tlsph_force<D, T, K, true> over packed records (same terms, same operation order, so
-// the same bits); one neighbour in flight per lane, which measured fastest with the wide loads.
+// the same bits); one neighbour in flight per lane, which measured fastest with the wide loads
+// (its record fills the registers).  The gathers bound it: 117 neighbours times 128 bytes for
+// each of 101^3 points are 15 GB through the caches.  The next neighbour's list entry is loaded
+// before this one's arithmetic, so that a step waits for one load and not for two in a row, and
+// larger workgroups share more lines (ListShape): pack included, Float32 927 -> 821 us, Float64
+// 1740 -> 1643 us.  Gathering whole records into LDS took 849 us and more (Float64 2.1 ms), one
+// array per 16-byte part 982 us.
 template <int D, class T, class K>
-__global__ __launch_bounds__(256) void k_list_tlsph_force_rec(const int32_t* __restrict__ row_ptr,
+__global__ __launch_bounds__((ListShape<T, true>::rec_threads)) void k_list_tlsph_force_rec(const int32_t* __restrict__ row_ptr,
                                                               const int32_t* __restrict__ col, int stored_base,
                                                               int64_t sel_first, const int32_t* __restrict__ sel_list,
                                                               int64_t n_sel, const uint4* __restrict__ rec,
@@ -671,7 +746,7 @@ __global__ __launch_bounds__(256) void k_list_tlsph_force_rec(const int32_t* __r
                                                               T* __restrict__ dv, int accumulate, int nblocks) {
     using RC = TlsphRec<D, T>;
     constexpr int LIST_LANES = ListShape<T, true>::lanes;
-    constexpr int LIST_ROWS_PER_BLOCK = ListShape<T, true>::rows;
+    constexpr int LIST_ROWS_PER_BLOCK = ListShape<T, true>::rec_threads / LIST_LANES;
     const int sub = threadIdx.x & (LIST_LANES - 1);
     const int64_t a = (int64_t)xcd_remap(blockIdx.x, nblocks) * LIST_ROWS_PER_BLOCK + (threadIdx.x / LIST_LANES);
     if (a >= n_sel) return;  // a row's lanes leave together
@@ -684,9 +759,11 @@ __global__ __launch_bounds__(256) void k_list_tlsph_force_rec(const int32_t* __r
     T acc[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) acc[d] = (T)0;
+    int64_t j = b + sub < e ? (int64_t)col[b + sub] - stored_base : 0;
     for (int k = b + sub; k < e; k += LIST_LANES) {
         T rj[RC::R];
-        load_rec<D, T>(rec, (int64_t)col[k] - stored_base, rj);
+        load_rec<D, T>(rec, j, rj);
+        if (k + LIST_LANES < e) j = (int64_t)col[k + LIST_LANES] - stored_base;
         T Xab[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) Xab[d] = ri[RC::X + d] - rj[RC::X + d];
