@@ -528,18 +528,27 @@ int check_queries(pn_grid& g, int queries, const BinSet*& Q) {
     return PN_OK;
 }
 
-// Whether the run kernels (pn_runs.h) take a traversal: they need a cell per sorted position
-// (a FullGridCellList), lengths that Float32 holds with room for their squares, and planes that a
-// 32-bit byte offset reaches.  They are faster than the cell kernel (k_cells) over the sizes
-// measured (1M points, F32: count 116 -> 90 us, density 236 -> 152, pressure 238 -> 177, TrixiParticles
-// interact! 623 -> 432, F64 1367 -> 831; 1000 points: count 14.7 -> 10.3, density 24.5 -> 15.7) but
-// for 2D pair functors below about 100,000 points (2000 points: density 7.6 -> 8.9 us) and for
-// counting an undeformed lattice whose search radius is a lattice distance (128^3, r = 3 spacings:
-// 305 -> 400 us, a quarter of the neighbours are ties), so the list builder counts by cells.
+// Whether the run kernels (pn_runs.h) take a traversal of n query points: they need a cell per
+// sorted position (a FullGridCellList), lengths that Float32 holds with room for their squares, and
+// planes that a 32-bit byte offset reaches.  They are faster than the cell kernel (k_cells) over the
+// sizes measured (1M points, F32: count 116 -> 90 us, density 236 -> 152, pressure 238 -> 177,
+// TrixiParticles interact! 623 -> 432, F64 1367 -> 831; 1000 points: count 14.7 -> 9.0, density
+// 24.5 -> 13) but for
+//   * queries that are sparse among the grid's points, whose runs are single points and take a
+//     wavefront's runs one after another (cells / runs, us, 512,000 points: n-body 1000 probes
+//     12 / 66, 30,000 41 / 55, 60,000 55 / 57, 120,000 72 / 61; count 21 / 41, 31 / 39, 38 / 41,
+//     44 / 46; 29,791 points: n-body 2000 probes 21 / 40, 8000 32 / 30): from one query for eight points on;
+//   * 2D pair functors over small clouds, whose cells have few candidates (density, r = 2.3 and 2.8
+//     spacings: 4200 points 7.2 / 8.1 and 7.7 / 8.5, 19,200 points 8.2 / 12.2 and 8.4 / 11, 90,000
+//     points 15.7 / 13.5 and 14.1 / 17): below 32,768 points;
+//   * counting an undeformed lattice whose search radius is a lattice distance (128^3, r = 3
+//     spacings: 305 -> 400 us, a quarter of the neighbours are ties): the list builder counts by cells.
 template <class F>
-bool runs_apply(const pn_grid& g) {
+bool runs_apply(const pn_grid& g, int64_t n) {
     if ((g.algorithm != 0 && !g.geom.periodic) || g.geom.hash || F::kFill) return false;
     if (g.grid.cap > (int64_t)1 << 28) return false;
+    if (8 * n < g.grid.n_sel) return false;
+    if (!F::kLight && g.nd == 2 && n < 32768 && !g.geom.periodic) return false;
     if (!(g.radius >= 0x1p-60 && g.radius <= 0x1p60)) return false;
     if (g.geom.periodic)
         for (int d = 0; d < g.nd; ++d)
@@ -567,6 +576,11 @@ void run_params(const pn_grid& g, int64_t n, bool known, bool light, bool fresh,
     const int64_t nc = g.grid.n_sel;
     const double work = n < nc ? (double)n * std::sqrt((double)n / (double)nc) : (double)n;
     sp.most = light ? (work >= 32768 ? 32 : (work >= 8192 ? 16 : 8)) : (work >= 65536 ? 32 : (work >= 24576 ? 16 : 8));
+    // A window that crosses into the next x-row has two runs or more.  Where the launch leaves the
+    // chip idle, two wavefronts share them (us with one / two, r = 2.8 spacings: 4096 points count
+    // 13.1 / 11.8, density 18.2 / 17.0, interact! 26.2 / 22.3; 1000 points 16.8 / 14.0 and 24.5 / 19.7;
+    // 13,824 points 20.2 / 23.6 and 30.0 / 33.2).
+    sp.lg_parts = (n + sp.most - 1) / sp.most <= 576 ? 1 : 0;
     sp.span = pn::RUN_SPAN;
     sp.magic0 = 0xffffffffu / (unsigned)geom.n[0];
     sp.magic1 = 0xffffffffu / (unsigned)geom.n[1];
@@ -595,7 +609,7 @@ int launch_runs(pn_grid& g, const BinSet* Q, const F& f) {
     pn::RunScale sc;
     pn::RunSplit sp;
     run_params(g, n, Q->stats_known, F::kLight, g.grid.fresh, sc, sp);
-    const int nblocks = (int)std::min<int64_t>(round_up8((n + sp.most - 1) / sp.most), g.persist_blocks);
+    const int nblocks = (int)std::min<int64_t>(round_up8((n + sp.most - 1) / sp.most << sp.lg_parts), g.persist_blocks);
     LaunchTimer timer(g);  // brackets the one traversal kernel launched below
     auto launch = [&](auto perc) {
         constexpr bool PER = decltype(perc)::value;
@@ -632,7 +646,7 @@ int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* 
         f.fstride = stride;
     }
     if constexpr (!F::kFill) {
-        if (allow_runs && runs_apply<F>(g)) return launch_runs<D, TC, TR, F>(g, Q, f);
+        if (allow_runs && runs_apply<F>(g, Q->stats_known ? Q->stats.n_binned : Q->n_sel)) return launch_runs<D, TC, TR, F>(g, Q, f);
     }
     // Upper bound on non-empty query cells; the kernel reads the exact count on device.
     int64_t nwork = std::min<int64_t>(g.geom.ncells, Q->n_sel);

@@ -40,9 +40,12 @@ namespace pn {
 
 constexpr int RUN = 32;       // most queries of a run
 constexpr int RUN_SPAN = 32;  // cells in x that a run may cover: keeps the split values in range
-// A run ends where the next query is this many cells further in x: from there on two runs stage
-// fewer candidates than one.
-constexpr int RUN_GAP = 4;
+// A run ends where the next query is this many cells further in x.  Two runs stage fewer candidates
+// than one from a gap of 4 cells on, but each starts with a chain of loads of some 5 us: at 4, the
+// few points of a thin row made a small cloud wait for eight runs of one (19,200 points in 2D, r = 2.3
+// spacings: interact! 21 -> 13 us, count 13.3 -> 9.2; 90,000 at r = 2.8: 25.4 -> 21.0; without such
+// rows the same).
+constexpr int RUN_GAP = 12;
 constexpr float PREFILTER_EPS = 3.8146973e-06f;  // 2^-18
 // Squared lengths that decide a pair alone: "certainly not" and "maybe" (|x|^2 stays below 1500,
 // and REJECT + MAYBE < 0).
@@ -61,6 +64,7 @@ struct RunScale {
 struct RunSplit {
     int n;     // points of the query set, -1: read on the device
     int most;  // queries of a run, a power of two up to RUN
+    int lg_parts;  // 2^lg_parts wavefronts share the runs of a window of `most` positions
     int span;  // cells of a run
     unsigned magic0, magic1;  // floor((2^32 - 1) / cells) in x and y (no batch table)
     int cell64;  // cells are computed in Float64
@@ -96,11 +100,14 @@ __device__ __forceinline__ unsigned div_magic(unsigned x, unsigned n, unsigned m
     return x - q * n >= n ? q + 1 : q;
 }
 
-// Calls fn(RunDesc) for the runs of the window of `most` (at most RUN) sorted positions from p0: it
-// is cut where the x-row changes, where a run would cover more than `span` cells and at gaps.
+// Calls fn(RunDesc) for the runs of work item w, the window of `most` (at most RUN) sorted positions
+// from (w >> lg_parts) * most: it is cut where the x-row changes, where a run would cover more than
+// `span` cells and at gaps.  The window's work items take its runs in turn.
 template <int D, class Fn>
-__device__ __forceinline__ void for_runs(const Geom& g, const SetView& Q, int p0, int n, const RunSplit& sp, Fn&& fn) {
+__device__ __forceinline__ void for_runs(const Geom& g, const SetView& Q, int w, int n, const RunSplit& sp, Fn&& fn) {
     const int lane = threadIdx.x;
+    const int p0 = (w >> sp.lg_parts) * sp.most, mask = (1 << sp.lg_parts) - 1;
+    int turn = w & mask;
     const int cnt = min(sp.most, n - p0);
     const int key_l = Q.keys[p0 + min(lane, cnt - 1)];
     const int step = key_l - __shfl_up(key_l, 1, WAVE);
@@ -135,7 +142,8 @@ __device__ __forceinline__ void for_runs(const Geom& g, const SetView& Q, int p0
         rd.q0 = p0 + i;
         rd.nq = end - i;
         rd.cb = __builtin_amdgcn_readlane(cx, end - 1);
-        fn(rd);
+        if (turn == 0) fn(rd);
+        turn = (turn - 1) & mask;
         i = end;
     }
 }
@@ -490,12 +498,12 @@ __global__ __launch_bounds__(WAVE, 4) void k_runs_count(Geom g, SetView Q, SetVi
     for (int d = 0; d < D; ++d) box[d] = (TR)g.box[d];
     const TR r2_in = r2 - r2 * (TR)sc.cell_rel;  // up to this x distance squared cells are adjacent
     const int n = sp.n >= 0 ? sp.n : Q.st->n_binned;
-    const int n_work = (n + sp.most - 1) / sp.most;
+    const int n_work = (n + sp.most - 1) / sp.most << sp.lg_parts;
     const int xcd = blockIdx.x & 7, per_xcd = nblocks >> 3;
     const int wchunk = (n_work + 7) >> 3;
     const int w_end = min(n_work, (xcd + 1) * wchunk);
     for (int w = xcd * wchunk + (int)(blockIdx.x >> 3); w < w_end; w += per_xcd) {
-        for_runs<D>(g, Q, w * sp.most, n, sp, [&](const RunDesc& rd) {
+        for_runs<D>(g, Q, w, n, sp, [&](const RunDesc& rd) {
             const RunLanes ln(rd.nq);
             const bool qact = ln.query < rd.nq;
             const int qpos = rd.q0 + (qact ? ln.query : 0);
@@ -682,12 +690,12 @@ __global__ __launch_bounds__(WAVE, (sizeof(TR) == 8 ? 3 : 4)) void k_runs(Geom g
     for (int d = 0; d < D; ++d) box[d] = (TR)g.box[d];
     const TR r2_in = r2 - r2 * (TR)sc.cell_rel;  // up to this x distance squared cells are adjacent
     const int n = sp.n >= 0 ? sp.n : Q.st->n_binned;
-    const int n_work = (n + sp.most - 1) / sp.most;
+    const int n_work = (n + sp.most - 1) / sp.most << sp.lg_parts;
     const int xcd = blockIdx.x & 7, per_xcd = nblocks >> 3;
     const int wchunk = (n_work + 7) >> 3;
     const int w_end = min(n_work, (xcd + 1) * wchunk);
     for (int w = xcd * wchunk + (int)(blockIdx.x >> 3); w < w_end; w += per_xcd) {
-        for_runs<D>(g, Q, w * sp.most, n, sp, [&](const RunDesc& rd) {
+        for_runs<D>(g, Q, w, n, sp, [&](const RunDesc& rd) {
             const RunLanes ln(rd.nq);
             const bool qact = ln.query < rd.nq;
             const int qpos = rd.q0 + (qact ? ln.query : 0);
