@@ -1,5 +1,6 @@
 // C-ABI traversal entry points: neighbour counts, index sums and CSR neighbour lists.
 #include "pn_host.h"
+#include "pn_fill.h"
 extern "C" {
 
 int pn_count_neighbors(pn_grid_t grid, int queries, int32_t* counts, int accumulate) {
@@ -31,7 +32,9 @@ int pn_csr_count(pn_grid_t grid, int queries, int64_t n_rows, int32_t* row_ptr, 
     if (n_rows < Q->n_src) return fail(PN_ERR_ARGUMENT, "n_rows is smaller than the number of query points");
     if (n_rows > INT32_MAX - 1) return fail(PN_ERR_ARGUMENT, "too many rows");
     int rc;
-    if ((rc = g.csr_counts.ensure((size_t)std::max<int64_t>(n_rows, 1) * 4, g.stream))) return rc;
+    // the fill keeps the positions of the grid's points there once the counts are summed
+    const int64_t n_counts = std::max(n_rows, std::max<int64_t>(g.grid.n_src, 1));
+    if ((rc = g.csr_counts.ensure((size_t)n_counts * 4, g.stream))) return rc;
     if ((rc = g.csr_status.ensure(sizeof(pn::DevStatus), g.stream))) return rc;
     if (!g.csr_host_status)
         PN_HIP(hipHostMalloc((void**)&g.csr_host_status, sizeof(pn::DevStatus), hipHostMallocDefault));
@@ -59,6 +62,20 @@ int pn_csr_count(pn_grid_t grid, int queries, int64_t n_rows, int32_t* row_ptr, 
     return PN_OK;
 }
 
+// Whether k_fill_sorted makes the lists of the queries: a FullGridCellList without a box or a
+// batch, whose fullest cell bounds a cell's candidates by what the kernel sorts in registers.  It
+// shares a cell's sorted candidates among the cell's queries, so it needs many of them: 3D from 12
+// points a cell on (k_cells and sort / k_fill_sorted, us, a million points F32: 7.5 a cell 294 / 315, 10
+// a cell 310 / 347; 216,000 points with 14 a cell 120 / 104; 2D with 16 a cell 196 / 203), and enough
+// cells to fill the chip (r = 3 spacings: 27,000 points 55 / 62, 125,000 points 90 / 86, F64 126 / 101).
+static bool fill_sorted_applies(const pn_grid& g, const BinSet& Q) {
+    const BinSet& G = g.grid;
+    if (g.nd != 3 || g.algorithm != 0 || g.geom.hash || g.geom.periodic || g.geom.table) return false;
+    if (!G.stats_known || (size_t)G.n_src * 4 > g.csr_counts.bytes) return false;
+    if (G.stats.n_binned < 100000 || G.stats.n_binned / 12 < G.stats.n_nonempty || Q.n_sel < G.n_sel) return false;
+    return 27 * (int64_t)G.stats.max_count <= pn::FILL_CAP;
+}
+
 int pn_csr_fill(pn_grid_t grid, int queries, int64_t n_rows, const int32_t* row_ptr, int32_t* col_idx,
                 int index_base) {
     if (!grid) return fail(PN_ERR_ARGUMENT, "grid is NULL");
@@ -69,6 +86,31 @@ int pn_csr_fill(pn_grid_t grid, int queries, int64_t n_rows, const int32_t* row_
     if (n_rows < Q->n_src) return fail(PN_ERR_ARGUMENT, "n_rows is smaller than the number of query points");
     if (g.csr_host_status && g.csr_host_status->max_count > pn::SORT_CAP)
         return fail(PN_ERR_UNSUPPORTED, "neighbor lists longer than 4096 entries are not supported");
+    if (fill_sorted_applies(g, *Q)) {
+        auto* inv = g.csr_counts.as<int32_t>();
+        hipLaunchKernelGGL(pn::k_invert, dim3(blocks_for(g.grid.n_sel, 256)), dim3(256), 0, g.stream,
+                           g.grid.sorted_idx.as<int32_t>(), g.grid.status.as<pn::DevStatus>(), inv);
+        PN_CHECK_LAUNCH();
+        const int64_t nwork = Q->stats_known ? Q->stats.n_nonempty : std::min<int64_t>(g.geom.ncells, Q->n_sel);
+        const int nblocks = (int)std::min<int64_t>(round_up8(std::max<int64_t>(nwork, 1)), g.persist_blocks);
+        // at least a cell's candidates; the network sorts 64 times a power of two keys
+        int n_keys = 4 * pn::WAVE;
+        while (n_keys < 27 * (int)g.grid.stats.max_count) n_keys *= 2;
+        const pn::FillArgs a{inv, row_ptr, col_idx, index_base};
+        LaunchTimer timer(g);  // brackets the one traversal kernel launched below
+        return dispatch_trav(g, [&](auto dc, auto tcv, auto trv) -> int {
+            if constexpr (decltype(dc)::value == 3) {
+                using TC = decltype(tcv);
+                using TR = decltype(trv);
+                const TR r = (TR)g.radius;
+                hipLaunchKernelGGL((pn::k_fill_sorted<3, TC, TR>), dim3(nblocks), dim3(pn::WAVE),
+                                   n_keys * sizeof(int), g.stream, g.geom, Q->view(), g.grid.view(), r * r, a, n_keys,
+                                   nblocks);
+                PN_CHECK_LAUNCH();
+            }
+            return PN_OK;
+        });
+    }
     pn::FillF f;
     f.row_ptr = row_ptr;
     f.col = col_idx;
