@@ -80,10 +80,13 @@ struct DevStatus {
     int n_nonempty;                // number of non-empty cells
     int n_binned;                  // number of binned points (low 32 bits of the sum)
     int n_ordered;                 // work items appended by k_order_work
+    // k_bin's minimum, moved to first_bad and set back to ~0 by the scan, so that the next binning
+    // finds it ready without a launch of its own
+    unsigned long long bad_now;
 };
 
-// Host copy of a binning's status in pinned, coherent host memory.  k_scan_top, the last
-// kernel of a binning to change the fields the host checks, stores the status there and
+// Host copy of a binning's status in pinned, coherent host memory.  The scan (or k_build_small),
+// the last of a binning to change the fields the host checks, stores the status there and
 // then raises `seq` with a system-scope release, so the host can raise the binning's
 // errors while the scatter and the in-cell ordering still run.
 struct StatusMailbox {
@@ -127,6 +130,7 @@ static __global__ void k_reset_status(DevStatus* st) {
     st->n_nonempty = 0;
     st->n_binned = 0;
     st->n_ordered = 0;
+    st->bad_now = ~0ull;
 }
 
 static __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
@@ -241,6 +245,21 @@ __device__ __forceinline__ int64_t sel_point(int64_t a, int64_t sel_first, const
     return sel_list ? (int64_t)sel_list[a] : sel_first + a;
 }
 
+// 0-based cell of point p (ok: it lies in the grid).
+template <int D, class TC, class TCELL>
+__device__ __forceinline__ int point_key(const Geom& g, const TC* __restrict__ y, int64_t p, bool& ok) {
+    if (g.hash) {
+        int64_t c[3];
+        hash_cell<D, TC, TCELL>(g, y + (int64_t)D * p, c, ok);
+        return spatial_hash<D>(c, g);
+    }
+    if (g.table) {
+        const GeomEntry e = g.table[g.cloud_of_point[p]];
+        return e.cell_off + cell_key<D, TC, TCELL>(e.n, e.minc, g.csd, g, y + (int64_t)D * p, ok);
+    }
+    return cell_key<D, TC, TCELL>(g.n, g.minc, g.csd, g, y + (int64_t)D * p, ok);
+}
+
 // One thread per selected point.  Lanes of a wavefront whose keys form a run (common:
 // inputs are usually close to cell order) share one atomic on the histogram; the slot
 // of each point inside its cell segment is the atomic's old value plus its run offset.
@@ -255,19 +274,9 @@ __global__ __launch_bounds__(256) void k_bin(Geom g, const TC* __restrict__ y, i
     if (a < n_sel) {
         int64_t p = sel_point(a, sel_first, sel_list);
         bool ok;
-        int k;
-        if (g.hash) {
-            int64_t c[3];
-            hash_cell<D, TC, TCELL>(g, y + (int64_t)D * p, c, ok);
-            k = spatial_hash<D>(c, g);
-        } else if (g.table) {
-            const GeomEntry e = g.table[g.cloud_of_point[p]];
-            k = e.cell_off + cell_key<D, TC, TCELL>(e.n, e.minc, g.csd, g, y + (int64_t)D * p, ok);
-        } else {
-            k = cell_key<D, TC, TCELL>(g.n, g.minc, g.csd, g, y + (int64_t)D * p, ok);
-        }
+        const int k = point_key<D, TC, TCELL>(g, y, p, ok);
         if (ok) key = k;
-        else atomicMin(&st->first_bad, (unsigned long long)a);
+        else atomicMin(&st->bad_now, (unsigned long long)a);
         keys[a] = key;
     }
     const int prev = __shfl_up(key, 1, WAVE);
@@ -303,9 +312,8 @@ __device__ __forceinline__ unsigned long long wave_incl_scan(unsigned long long 
     return v;
 }
 
-// Block-wide exclusive scan of one value per thread (256 threads = 4 waves).
-__device__ __forceinline__ unsigned long long block_excl_scan(unsigned long long v,
-                                                              unsigned long long* sh /*4*/,
+// Block-wide exclusive scan of one value per thread (sh: one entry per wave).
+__device__ __forceinline__ unsigned long long block_excl_scan(unsigned long long v, unsigned long long* sh,
                                                               unsigned long long& total) {
     const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x >> 6;
     unsigned long long inc = wave_incl_scan(v, lane);
@@ -355,6 +363,25 @@ static __global__ __launch_bounds__(SCAN_THREADS) void k_scan_reduce(const int32
     }
 }
 
+// The status of a binning whose packed counts sum to `sum`; in pinned host memory too when mb.
+__device__ __forceinline__ void publish_status(DevStatus* st, StatusMailbox* mb, unsigned long long seq,
+                                               unsigned long long bad, unsigned long long total64, int max_count,
+                                               unsigned long long sum) {
+    DevStatus s;
+    s.first_bad = bad;
+    s.total64 = total64;
+    s.max_count = max_count;
+    s.n_nonempty = (int)(uint32_t)(sum >> 32);
+    s.n_binned = (int)(uint32_t)(sum & 0xffffffffull);
+    s.n_ordered = 0;
+    s.bad_now = ~0ull;
+    *st = s;
+    if (mb) {
+        mb->status = s;
+        __hip_atomic_store(&mb->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // Single workgroup: exclusive scan of the block sums (block_sums[0, nblocks)), writes the
 // totals, the 64-bit sum of all counts and the largest count (block maxima at
 // block_sums[nblocks, 2 nblocks)).
@@ -397,21 +424,8 @@ static __global__ __launch_bounds__(SCAN_THREADS) void k_scan_top(unsigned long 
             tot += sh_sum[i];
             m = max(m, sh_max[i]);
         }
-        st->total64 = tot;
-        st->max_count = m;
         start[C] = (int32_t)(uint32_t)(carry & 0xffffffffull);
-        st->n_binned = (int)(uint32_t)(carry & 0xffffffffull);
-        st->n_nonempty = (int)(uint32_t)(carry >> 32);
-        if (mb) {
-            // first_bad comes from k_bin, an earlier kernel on the same stream
-            mb->status.first_bad = st->first_bad;
-            mb->status.total64 = tot;
-            mb->status.max_count = m;
-            mb->status.n_nonempty = (int)(uint32_t)(carry >> 32);
-            mb->status.n_binned = (int)(uint32_t)(carry & 0xffffffffull);
-            mb->status.n_ordered = 0;
-            __hip_atomic_store(&mb->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
+        publish_status(st, mb, seq, st->bad_now, tot, m, carry);  // bad_now: of k_bin, an earlier kernel
     }
 }
 
@@ -527,6 +541,186 @@ __global__ __launch_bounds__(256) void k_canon(const int32_t* __restrict__ keys,
     sorted_keys[c.pos] = c.key;
 #pragma unroll
     for (int d = 0; d < D; ++d) coords[(int64_t)d * cap + c.pos] = y[(int64_t)D * c.p + d];
+}
+
+// The whole scan of up to SCAN_ONE_MAX counts, which it leaves zero, in one workgroup: what
+// k_scan_reduce, k_scan_top and k_scan_down do in three launches of 3 to 6 us, most of it the launch
+// (1900 cells 10 us and two gaps, here 5; 15,000 cells 12 us, here 7; the time grows by the 64 rows
+// of cells that a wavefront takes, so the chip's three passes win beyond).
+constexpr int BUILD_THREADS = 1024;
+constexpr int SCAN_ONE_ITEMS = 16;
+constexpr int SCAN_ONE_MAX = BUILD_THREADS * SCAN_ONE_ITEMS;
+
+// Inclusive sums over the wavefront's lanes (DPP row shifts and broadcasts).
+__device__ __forceinline__ int wave_incl_scan_dpp(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+
+// Exclusive sums of a workgroup's C counts, count(c), into put(c, first, rank among the non-empty,
+// count); returns the packed sum and sets the largest count.  A wavefront takes consecutive rows of
+// 64 cells, so that its loads and stores are whole lines.
+template <class Count, class Put>
+__device__ __forceinline__ unsigned long long scan_one(int C, unsigned long long* sh, int* sh_max, int& max_count,
+                                                       Count&& count, Put&& put) {
+    const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x >> 6;
+    const int rows = (C + BUILD_THREADS - 1) / BUILD_THREADS;  // of each wavefront, at most SCAN_ONE_ITEMS
+    const int c0 = w * rows * WAVE + lane;
+    int v[SCAN_ONE_ITEMS];
+#pragma unroll
+    for (int i = 0; i < SCAN_ONE_ITEMS; ++i) v[i] = i < rows && c0 + i * WAVE < C ? count(c0 + i * WAVE) : 0;
+    unsigned long long s = 0;
+    int mx = 0;
+#pragma unroll
+    for (int i = 0; i < SCAN_ONE_ITEMS; ++i) {
+        s += pack_cell(v[i]);
+        mx = max(mx, v[i]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        s += __shfl_xor(s, o, WAVE);
+        mx = max(mx, __shfl_xor(mx, o, WAVE));
+    }
+    if (lane == 0) {
+        sh[w] = s;
+        sh_max[w] = mx;
+    }
+    __syncthreads();
+    unsigned long long before = 0, total = 0;
+    max_count = 0;
+#pragma unroll
+    for (int i = 0; i < BUILD_THREADS / WAVE; ++i) {
+        before += i < w ? sh[i] : 0ull;
+        total += sh[i];
+        max_count = max(max_count, sh_max[i]);
+    }
+    int first = (int)(uint32_t)(before & 0xffffffffull), rank = (int)(uint32_t)(before >> 32);
+#pragma unroll
+    for (int i = 0; i < SCAN_ONE_ITEMS; ++i) {
+        if (i >= rows) break;
+        const int incl = wave_incl_scan_dpp(v[i]);
+        const unsigned long long some = __ballot(v[i] > 0);
+        const int r = rank + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(some >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((unsigned)some, 0));
+        if (c0 + i * WAVE < C) put(c0 + i * WAVE, first + incl - v[i], r, v[i]);
+        first += __builtin_amdgcn_readlane(incl, WAVE - 1);
+        rank += __popcll(some);
+    }
+    return total;
+}
+
+static __global__ __launch_bounds__(BUILD_THREADS) void k_scan_one(int32_t* __restrict__ counts, int C,
+                                                            int32_t* __restrict__ start,
+                                                            int32_t* __restrict__ nonempty, DevStatus* st,
+                                                            StatusMailbox* mb, unsigned long long seq) {
+    __shared__ unsigned long long sh[BUILD_THREADS / WAVE];
+    __shared__ int sh_max[BUILD_THREADS / WAVE];
+    int max_count;
+    const unsigned long long sum = scan_one(
+        C, sh, sh_max, max_count, [&](int c) { return counts[c]; },
+        [&](int c, int first, int rank, int n) {
+            start[c] = first;
+            counts[c] = 0;
+            if (n > 0) nonempty[rank] = c;
+        });
+    if (threadIdx.x == 0) {
+        start[C] = (int32_t)(uint32_t)(sum & 0xffffffffull);
+        publish_status(st, mb, seq, st->bad_now, sum & 0xffffffffull, max_count, sum);
+    }
+}
+
+// A whole binning (k_bin, the scan, k_scatter and k_canon, in that order below) of up to
+// BUILD_SMALL_POINTS points in up to BUILD_SMALL_CELLS cells in one workgroup, the histogram and the
+// provisional placement in LDS: the launches cost more than their work there.  2000 points in 2D:
+// 24 us in seven kernels and the gaps between them become 9 us; 3375 points in 3D 14.5 us.  One
+// compute unit's loads and stores bound it: of 15,600 points the four kernels take 19 us.
+constexpr int BUILD_ITEMS = 4;
+constexpr int BUILD_SMALL_POINTS = BUILD_THREADS * BUILD_ITEMS;
+constexpr int BUILD_SMALL_CELLS = 11 * 1024;  // 64 KB of LDS
+
+template <int D, class TC, class TCELL>
+__global__ __launch_bounds__(BUILD_THREADS) void k_build_small(Geom g, const TC* __restrict__ y, int64_t sel_first,
+                                                               const int32_t* __restrict__ sel_list, int n_sel,
+                                                               int32_t* __restrict__ start,
+                                                               int32_t* __restrict__ nonempty,
+                                                               int32_t* __restrict__ sorted_idx,
+                                                               int32_t* __restrict__ sorted_keys,
+                                                               TC* __restrict__ coords, int64_t cap, int canonical,
+                                                               DevStatus* st, StatusMailbox* mb,
+                                                               unsigned long long seq) {
+    __shared__ int s_cell[BUILD_SMALL_CELLS + 1];  // counts, then starts
+    __shared__ int s_perm[BUILD_SMALL_POINTS];
+    __shared__ unsigned long long sh[BUILD_THREADS / WAVE];
+    __shared__ int sh_max[BUILD_THREADS / WAVE];
+    __shared__ int s_bad;
+    const int C = g.ncells;
+    for (int c = threadIdx.x; c < C; c += BUILD_THREADS) s_cell[c] = 0;
+    if (threadIdx.x == 0) s_bad = INT32_MAX;
+    __syncthreads();
+    int key[BUILD_ITEMS], slot[BUILD_ITEMS];
+    int32_t p[BUILD_ITEMS];
+#pragma unroll
+    for (int i = 0; i < BUILD_ITEMS; ++i) {
+        const int a = (int)threadIdx.x + i * BUILD_THREADS;
+        key[i] = -1;
+        if (a < n_sel) {
+            p[i] = (int32_t)sel_point(a, sel_first, sel_list);
+            bool ok;
+            const int k = point_key<D, TC, TCELL>(g, y, p[i], ok);
+            if (ok) {
+                key[i] = k;
+                slot[i] = atomicAdd(&s_cell[k], 1);
+            } else {
+                atomicMin(&s_bad, a);
+            }
+        }
+    }
+    __syncthreads();
+    int max_count;
+    const unsigned long long sum = scan_one(
+        C, sh, sh_max, max_count, [&](int c) { return s_cell[c]; },
+        [&](int c, int first, int rank, int n) {
+            s_cell[c] = first;
+            start[c] = first;
+            if (n > 0) nonempty[rank] = c;
+        });
+    if (threadIdx.x == 0) {
+        s_cell[C] = start[C] = (int32_t)(uint32_t)(sum & 0xffffffffull);
+        publish_status(st, mb, seq, s_bad == INT32_MAX ? ~0ull : (unsigned long long)s_bad, sum & 0xffffffffull,
+                       max_count, sum);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < BUILD_ITEMS; ++i)
+        if (key[i] >= 0) s_perm[s_cell[key[i]] + slot[i]] = (int)threadIdx.x + i * BUILD_THREADS;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < BUILD_ITEMS; ++i) {
+        if (key[i] < 0) continue;
+        const int a = (int)threadIdx.x + i * BUILD_THREADS, b = s_cell[key[i]], e = s_cell[key[i] + 1];
+        int pos = b + slot[i];
+        if (canonical && e - b <= CANON_RANK_LIMIT) {
+            pos = b;
+            for (int q = b; q < e; ++q) {
+                const int aq = s_perm[q];
+                if (!sel_list) {
+                    pos += aq < a;
+                } else {
+                    const int32_t pq = sel_list[aq];
+                    pos += (pq < p[i]) || (pq == p[i] && aq < a);
+                }
+            }
+        }
+        sorted_idx[pos] = p[i];
+        sorted_keys[pos] = key[i];
+#pragma unroll
+        for (int d = 0; d < D; ++d) coords[(int64_t)d * cap + pos] = y[(int64_t)D * p[i] + d];
+    }
 }
 
 // k_canon for a SpatialHashingCellList, which also records the bucket data the cell kernel

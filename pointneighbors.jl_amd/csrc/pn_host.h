@@ -80,6 +80,12 @@ struct Scanner {
     int run(const int32_t* counts, int64_t n, int32_t* start, int32_t* nonempty, pn::DevStatus* st,
             hipStream_t stream, pn::StatusMailbox* mb = nullptr, unsigned long long seq = 0,
             bool clear_counts = false) {
+        if (clear_counts && n <= pn::SCAN_ONE_MAX) {
+            hipLaunchKernelGGL(pn::k_scan_one, dim3(1), dim3(pn::BUILD_THREADS), 0, stream,
+                               const_cast<int32_t*>(counts), (int)n, start, nonempty, st, mb, seq);
+            PN_CHECK_LAUNCH();
+            return PN_OK;
+        }
         const int64_t nb = std::max<int64_t>(1, (n + pn::SCAN_TILE - 1) / pn::SCAN_TILE);
         int rc = block_sums.ensure((size_t)nb * 16, stream);  // block sums, then block maxima
         if (rc) return rc;
@@ -104,7 +110,7 @@ struct BinSet {
     Buf bucket_cell, bucket_mixed;  // SpatialHashingCellList: per-bucket cell and collision flag
     int hash_epoch = 0;             // bucket_mixed value of a mixed bucket of the last binning
     pn::DevStatus* host_status = nullptr;  // pinned
-    // pinned coherent host memory k_scan_top publishes the status to; mail_seq is the
+    // pinned coherent host memory the scan publishes the status to; mail_seq is the
     // sequence number of the last binning that asked for it
     pn::StatusMailbox* mailbox = nullptr;
     unsigned long long mail_seq = 0;
@@ -112,6 +118,7 @@ struct BinSet {
     bool mailbox_failed = false;  // its allocation failed once: not tried again
     Scanner scan;
     bool counts_zero = false;  // `counts` holds zeros (left so by the last binning's scan)
+    bool status_ready = false;  // `status` is as the last binning's scan left it
     int64_t cap = 0;
     int64_t n_sel = 0;        // selected points of the last binning
     int64_t n_src = 0;        // columns of the source matrix
@@ -245,7 +252,9 @@ int ensure_set(pn_grid& g, BinSet& s, int64_t n_sel) {
     if (s.counts.p != counts_before) s.counts_zero = false;
     if ((rc = s.start.ensure((size_t)(C + 1) * 4, g.stream))) return rc;
     if ((rc = s.nonempty.ensure((size_t)C * 4, g.stream))) return rc;
+    const void* status_before = s.status.p;
     if ((rc = s.status.ensure(sizeof(pn::DevStatus), g.stream))) return rc;
+    if (s.status.p != status_before) s.status_ready = false;
     if (g.geom.hash) {
         if ((rc = s.bucket_cell.ensure((size_t)C * 12, g.stream))) return rc;
         const size_t before = s.bucket_mixed.bytes;
@@ -326,18 +335,31 @@ int enqueue_bin(pn_grid& g, BinSet& s, const void* src, int64_t n_src, int64_t s
     auto* st = s.status.as<pn::DevStatus>();
     ++s.mail_seq;  // a new number for every binning enqueued, also one that fails below
     s.mail_pending = false;
-    hipLaunchKernelGGL(pn::k_reset_status, dim3(1), dim3(1), 0, g.stream, st);
-    PN_CHECK_LAUNCH();
-    if (!s.counts_zero) {
+    const bool small = !g.geom.hash && sel_count <= pn::BUILD_SMALL_POINTS && C <= pn::BUILD_SMALL_CELLS;
+    if (!s.status_ready && !small) {
+        hipLaunchKernelGGL(pn::k_reset_status, dim3(1), dim3(1), 0, g.stream, st);
+        PN_CHECK_LAUNCH();
+    }
+    s.status_ready = false;  // until this binning's scan is enqueued
+    if (!s.counts_zero && !small) {
         hipLaunchKernelGGL(pn::k_fill_i32, dim3(blocks_for(std::min<int64_t>(C, 1 << 20), 256)), dim3(256), 0,
                            g.stream, s.counts.as<int32_t>(), C, 0);
         PN_CHECK_LAUNCH();
     }
-    s.counts_zero = false;  // until this binning's scan is enqueued
+    if (!small) s.counts_zero = false;  // until this binning's scan is enqueued
     rc = dispatch_build(g, [&](auto dc, auto tcv, auto tcellv) -> int {
         constexpr int D = decltype(dc)::value;
         using TC = decltype(tcv);
         using TCELL = decltype(tcellv);
+        if (small) {
+            hipLaunchKernelGGL((pn::k_build_small<D, TC, TCELL>), dim3(1), dim3(pn::BUILD_THREADS), 0, g.stream, g.geom,
+                               (const TC*)src, sel_first, sel_list, (int)sel_count, s.start.as<int32_t>(),
+                               s.nonempty.as<int32_t>(), s.sorted_idx.as<int32_t>(), s.slots.as<int32_t>(),
+                               s.coords.as<TC>(), s.cap, g.canonical_order, st, s.mailbox, s.mail_seq);
+            PN_CHECK_LAUNCH();
+            s.status_ready = true;
+            return PN_OK;
+        }
         if (sel_count > 0) {
             hipLaunchKernelGGL((pn::k_bin<D, TC, TCELL>), dim3(blocks_for(sel_count, 256)), dim3(256), 0, g.stream,
                                g.geom, (const TC*)src, sel_first, sel_list, sel_count, s.keys.as<int32_t>(),
@@ -348,6 +370,7 @@ int enqueue_bin(pn_grid& g, BinSet& s, const void* src, int64_t n_src, int64_t s
                              g.stream, s.mailbox, s.mail_seq, true);
         if (rc2) return rc2;
         s.counts_zero = true;
+        s.status_ready = true;
         if (sel_count > 0) {
             // a hash build reuses `slots`, cleared to -1 here, for its bucket representatives
             hipLaunchKernelGGL(pn::k_scatter, dim3(blocks_for(sel_count, 256)), dim3(256), 0, g.stream,
@@ -440,7 +463,7 @@ int describe_point(pn_grid& g, const void* src, int64_t p) {
 }
 
 // The status of the last binning of s.  The mailbox path spins on the sequence number
-// k_scan_top raises (the host returns while the rest of the build still runs; a kernel
+// the scan raises (the host returns while the rest of the build still runs; a kernel
 // error after it surfaces at the next synchronization, as for any enqueued work); after
 // STATUS_SPIN_US without it, or with no mailbox, the status is copied after a stream
 // synchronization.
