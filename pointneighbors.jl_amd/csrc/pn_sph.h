@@ -280,7 +280,7 @@ struct DensityVjpF : FunctorBase {
         const T inv_r = prsqrt0(d2);
         const T r = d2 * inv_r;
         a.m = pfma(fj[1], kern.w(r), a.m);
-        const T c = (qs.g * fj[0] + fj[1] * qs.m) * kern.dw(r) * inv_r;
+        const T c = pfma(qs.g, fj[0], fj[1] * qs.m) * kern.dw(r) * inv_r;
 #pragma unroll
         for (int d = 0; d < D; ++d) a.x[d] = pfma(c, pd[d], a.x[d]);
     }
@@ -342,21 +342,22 @@ struct PressureVjpF : FunctorBase {
             const T w1 = kern.dw(r);
             const T w2 = kern.d2w(r);
             const T mj = fj[0], Pj = fj[1];
-            T v[D], u[D];
-            T vu = (T)0, abG = (T)0;
+            // with v = (x_i - x_j) / r and u = m_j abar_i - m_i abar_j:
+            //     x -= c (w2 (v.u) v + w1 / r (u - (v.u) v)) = c w1 / r u + c (w2 - w1 / r) (v.u) v
+            T u[D];
+            T ru = (T)0, rG = (T)0;  // r (v.u) and r (v.abar_j)
 #pragma unroll
             for (int d = 0; d < D; ++d) {
-                v[d] = pd[d] * inv_r;
-                u[d] = mj * qs.ab[d] - qs.m * fj[2 + d];
-                vu += v[d] * u[d];
-                abG += fj[2 + d] * v[d];
+                u[d] = pfma(mj, qs.ab[d], -(qs.m * fj[2 + d]));
+                ru = pfma(pd[d], u[d], ru);
+                rG = pfma(pd[d], fj[2 + d], rG);
             }
-            const T c = qs.P + Pj;
-            a.P -= w1 * vu;
-            a.m += c * w1 * abG;
-            const T wr = w1 * inv_r;
+            const T c = qs.P + Pj, wr = w1 * inv_r, vu = ru * inv_r;
+            a.P = pfma(-wr, ru, a.P);
+            a.m = pfma(c * wr, rG, a.m);
+            const T along = c * (wr - w2) * vu * inv_r, across = -(c * wr);
 #pragma unroll
-            for (int d = 0; d < D; ++d) a.x[d] -= c * (w2 * vu * v[d] + wr * (u[d] - vu * v[d]));
+            for (int d = 0; d < D; ++d) a.x[d] = pfma(along, pd[d], pfma(across, u[d], a.x[d]));
         }
     }
     __device__ void combine(Acc& a, const Acc& b) const {
