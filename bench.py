@@ -205,7 +205,7 @@ def main():
             trav_ms, kernel = dens_ms, "DensityF"
             # per neighbour: coordinates + m_j; out: rho_i
             algo = traversal_bytes(n, n_nonempty, f_in=4, f_own=0, f_out=4)
-    kernel = f"k_cells<3,float,float,{kernel}>"
+    kernel = "k_runs_count<3,float,float>" if kernel == "CountF" else f"k_runs<3,float,float,{kernel}>"
     achieved = algo / (trav_ms * 1e-3) / 1e9
 
     # measured HBM bytes per launch of this kernel (rocprofv3 FETCH_SIZE + WRITE_SIZE)

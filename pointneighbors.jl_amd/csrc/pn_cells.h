@@ -1,5 +1,7 @@
 // Candidate-major neighbour traversal (foreach_point_neighbor, hot loop
-// src/nhs_grid.jl:519-575) on gfx950: one wavefront per non-empty query cell.
+// src/nhs_grid.jl:519-575) on gfx950: one wavefront per non-empty query cell.  The run kernels
+// (pn_runs.h) take most traversals; this one has the hash lists, the list builder, sparse queries
+// and small 2D clouds.
 //
 // The 3^D cells around a query cell are 3^(D-1) x-rows of three adjacent cells, each a
 // contiguous range of the cell-sorted order.  The wavefront loads those candidates into

@@ -178,7 +178,7 @@ struct pn_grid {
     std::vector<int64_t> host_point_offsets;
     int64_t persist_blocks = 1 << 20;  // workgroups of the persistent traversal (multiple of 8)
     int chunk = 0;                  // candidate chunk: -1 per functor, 0 small, 1 large
-    int algorithm = 0;              // traversal: 0 candidate-major cells, 1 per-query slices
+    int algorithm = 0;              // traversal: 0 runs of queries or cells, 1 per-query slices
     int canonical_order = 1;        // 1: in-cell order = ascending original index
     Buf csr_counts;
     Buf csr_status;

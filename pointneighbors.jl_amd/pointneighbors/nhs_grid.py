@@ -227,8 +227,8 @@ class GridNeighborhoodSearch(metaclass=_GridMeta):
         return isinstance(self.cell_list, SpatialHashingCellList)
 
     def set_tuning(self, key, value):
-        """Autotuner knobs: "algorithm" (0: candidate-major cells, 1: per-query candidate
-        slices), "persist_blocks" (traversal workgroups, multiple of 8), "chunk" (-1 per
+        """Autotuner knobs: "algorithm" (0: runs of queries, or candidate-major cells where
+        those are faster, 1: per-query candidate slices), "persist_blocks" (traversal workgroups, multiple of 8), "chunk" (-1 per
         functor, 0 small, 1 large candidate chunk), "canonical_order" (1: in-cell order by
         original index; 0: atomic order, nondeterministic inside a cell)."""
         self._tuning[key] = int(value)
