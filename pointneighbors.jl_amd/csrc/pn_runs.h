@@ -24,7 +24,7 @@
 // coordinates moved without a new binning a run is one cell, so that the cells of the binning
 // decide, as in the reference.
 // Points for which the estimate cannot be trusted (a query outside its cell after an in-place
-// move, a candidate at a periodic box's half length) are kept as "maybe" for every pair.
+// move, a candidate whose other image in a periodic box may be as near) are kept as "maybe" for every pair.
 //
 // A run has up to 64 lanes for its queries: two per query, four for up to 16 and eight for up to
 // 8 queries, which share the query's candidates; their sums are combined in a fixed order, so
@@ -238,6 +238,7 @@ struct RunFrame {
     float hq[D];   // bound on |t_d| of the run's queries
     float hc[D];   // ... of the candidates that can be neighbours
     float len[D];  // periodic box
+    float near[D];  // ... up to this |t_d| a candidate's image is the nearest to every query within r
     float s, rt, per_mg;
 
     __device__ __forceinline__ void set(const Geom& g, const RunDesc& rd, const RunScale& sc) {
@@ -252,6 +253,10 @@ struct RunFrame {
             hq[d] = (float)(half * g.csd[d]) * s + 0.01f * rt;
             hc[d] = hq[d] + 1.01f * rt;
             len[d] = PER ? (float)g.box[d] * s : 0.0f;
+            // another image of a candidate at t is len - |t| from the centre, so at least
+            // len - |t| - hq from a query: further than r.  Half the length alone is not enough
+            // where the box has three cells.
+            near[d] = fminf(0.499f * len[d], len[d] - hq[d] - 1.01f * rt);
         }
     }
 
@@ -266,7 +271,7 @@ struct RunFrame {
                 const float l16 = 16.0f * len[d];
                 sure = sure && fabsf(t[d]) <= 4.0f * l16;
                 t[d] = __builtin_fmaf(-l16, rintf(t[d] / l16), t[d]);
-                sure = sure && fabsf(t[d]) <= 0.499f * l16;
+                sure = sure && fabsf(t[d]) <= 16.0f * near[d];
             }
         }
         return sure;
