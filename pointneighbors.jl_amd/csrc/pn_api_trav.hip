@@ -22,6 +22,33 @@ int pn_sum_neighbor_indices(pn_grid_t grid, int queries, int64_t* sums, int inde
     return launch_traverse(*grid, queries, f);
 }
 
+// Whether k_fill_sorted can make the lists of the queries: a 3D FullGridCellList without a box or a
+// batch, with enough points to fill the chip (r = 3 spacings, k_cells and sort / k_fill_sorted, us:
+// 27,000 points 55 / 62, 125,000 points 90 / 86, F64 126 / 101).
+static bool fill_sorted_possible(const pn_grid& g, const BinSet& Q) {
+    if (g.nd != 3 || g.algorithm != 0 || g.geom.hash || g.geom.periodic || g.geom.table) return false;
+    return g.grid.n_sel >= 100000 && Q.n_sel >= g.grid.n_sel;
+}
+
+// Whether it makes them, st being the grid's status: its fullest cell bounds a cell's candidates by
+// what the kernel sorts in registers.  It shares a cell's sorted candidates among the cell's queries,
+// so it needs many of them: from 12 points a cell on (us, a million points F32: 7.5 a cell 294 / 315,
+// 10 a cell 310 / 347; 216,000 points with 14 a cell 120 / 104; 2D with 16 a cell 196 / 203).
+static bool fill_sorted_applies(const pn::DevStatus& st) {
+    if (st.n_binned < 100000 || st.n_binned / 12 < st.n_nonempty) return false;
+    return 27 * (int64_t)st.max_count <= pn::FILL_CAP;
+}
+
+// Whether work is being captured on the stream (or may be: an implicit capture refuses the query).
+static bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return status != hipStreamCaptureStatusNone;
+}
+
 int pn_csr_count(pn_grid_t grid, int queries, int64_t n_rows, int32_t* row_ptr, int32_t max_neighbors,
                  int64_t* nnz, int64_t* max_row) {
     if (!grid) return fail(PN_ERR_ARGUMENT, "grid is NULL");
@@ -37,7 +64,7 @@ int pn_csr_count(pn_grid_t grid, int queries, int64_t n_rows, int32_t* row_ptr, 
     if ((rc = g.csr_counts.ensure((size_t)n_counts * 4, g.stream))) return rc;
     if ((rc = g.csr_status.ensure(sizeof(pn::DevStatus), g.stream))) return rc;
     if (!g.csr_host_status)
-        PN_HIP(hipHostMalloc((void**)&g.csr_host_status, sizeof(pn::DevStatus), hipHostMallocDefault));
+        PN_HIP(hipHostMalloc((void**)&g.csr_host_status, 2 * sizeof(pn::DevStatus), hipHostMallocDefault));
     auto* st = g.csr_status.as<pn::DevStatus>();
     hipLaunchKernelGGL(pn::k_reset_status, dim3(1), dim3(1), 0, g.stream, st);
     PN_CHECK_LAUNCH();
@@ -51,6 +78,13 @@ int pn_csr_count(pn_grid_t grid, int queries, int64_t n_rows, int32_t* row_ptr, 
     if ((rc = launch_traverse(g, queries, f, false))) return rc;
     if ((rc = g.csr_scan.run(g.csr_counts.as<int32_t>(), n_rows, row_ptr, nullptr, st, g.stream))) return rc;
     PN_HIP(hipMemcpyAsync(g.csr_host_status, st, sizeof(pn::DevStatus), hipMemcpyDeviceToHost, g.stream));
+    // the grid's own status from the device: the host's copy is that of an earlier binning where a
+    // captured one has been replayed
+    g.csr_grid_known = fill_sorted_possible(g, *Q);
+    g.csr_grid_seq = g.grid.mail_seq;
+    if (g.csr_grid_known)
+        PN_HIP(hipMemcpyAsync(g.csr_host_status + 1, g.grid.status.p, sizeof(pn::DevStatus), hipMemcpyDeviceToHost,
+                              g.stream));
     PN_HIP(hipStreamSynchronize(g.stream));
     const pn::DevStatus hs = *g.csr_host_status;
     if (nnz) *nnz = (int64_t)hs.total64;
@@ -60,20 +94,6 @@ int pn_csr_count(pn_grid_t grid, int queries, int64_t n_rows, int32_t* row_ptr, 
     if (max_neighbors > 0 && hs.max_count > max_neighbors)
         return fail(PN_ERR_LIST_FULL, "cell list is full. Use a larger `max_points_per_cell`.");
     return PN_OK;
-}
-
-// Whether k_fill_sorted makes the lists of the queries: a FullGridCellList without a box or a
-// batch, whose fullest cell bounds a cell's candidates by what the kernel sorts in registers.  It
-// shares a cell's sorted candidates among the cell's queries, so it needs many of them: 3D from 12
-// points a cell on (k_cells and sort / k_fill_sorted, us, a million points F32: 7.5 a cell 294 / 315, 10
-// a cell 310 / 347; 216,000 points with 14 a cell 120 / 104; 2D with 16 a cell 196 / 203), and enough
-// cells to fill the chip (r = 3 spacings: 27,000 points 55 / 62, 125,000 points 90 / 86, F64 126 / 101).
-static bool fill_sorted_applies(const pn_grid& g, const BinSet& Q) {
-    const BinSet& G = g.grid;
-    if (g.nd != 3 || g.algorithm != 0 || g.geom.hash || g.geom.periodic || g.geom.table) return false;
-    if (!G.stats_known || (size_t)G.n_src * 4 > g.csr_counts.bytes) return false;
-    if (G.stats.n_binned < 100000 || G.stats.n_binned / 12 < G.stats.n_nonempty || Q.n_sel < G.n_sel) return false;
-    return 27 * (int64_t)G.stats.max_count <= pn::FILL_CAP;
 }
 
 int pn_csr_fill(pn_grid_t grid, int queries, int64_t n_rows, const int32_t* row_ptr, int32_t* col_idx,
@@ -86,7 +106,11 @@ int pn_csr_fill(pn_grid_t grid, int queries, int64_t n_rows, const int32_t* row_
     if (n_rows < Q->n_src) return fail(PN_ERR_ARGUMENT, "n_rows is smaller than the number of query points");
     if (g.csr_host_status && g.csr_host_status->max_count > pn::SORT_CAP)
         return fail(PN_ERR_UNSUPPORTED, "neighbor lists longer than 4096 entries are not supported");
-    if (fill_sorted_applies(g, *Q)) {
+    // by the grid's status at pn_csr_count; a captured fill may be replayed over another binning
+    if (g.csr_grid_known && g.csr_grid_seq == g.grid.mail_seq && fill_sorted_possible(g, *Q) &&
+        fill_sorted_applies(g.csr_host_status[1]) && (size_t)g.grid.n_src * 4 <= g.csr_counts.bytes &&
+        !capturing(g.stream)) {
+        const int max_count = g.csr_host_status[1].max_count;
         auto* inv = g.csr_counts.as<int32_t>();
         hipLaunchKernelGGL(pn::k_invert, dim3(blocks_for(g.grid.n_sel, 256)), dim3(256), 0, g.stream,
                            g.grid.sorted_idx.as<int32_t>(), g.grid.status.as<pn::DevStatus>(), inv);
@@ -95,7 +119,7 @@ int pn_csr_fill(pn_grid_t grid, int queries, int64_t n_rows, const int32_t* row_
         const int nblocks = (int)std::min<int64_t>(round_up8(std::max<int64_t>(nwork, 1)), g.persist_blocks);
         // at least a cell's candidates; the network sorts 64 times a power of two keys
         int n_keys = 4 * pn::WAVE;
-        while (n_keys < 27 * (int)g.grid.stats.max_count) n_keys *= 2;
+        while (n_keys < 27 * max_count) n_keys *= 2;
         const pn::FillArgs a{inv, row_ptr, col_idx, index_base};
         LaunchTimer timer(g);  // brackets the one traversal kernel launched below
         return dispatch_trav(g, [&](auto dc, auto tcv, auto trv) -> int {

@@ -87,7 +87,7 @@ __global__ __launch_bounds__(WAVE, 6) void k_fill_sorted(Geom g, SetView Q, SetV
         rd.ca = rd.cb = cell - rd.row;
         RunPieces<D, false> pc;
         pc.set(g, Gs, rd);
-        pc.M = min(pc.M, n_keys);
+        pc.M = min(pc.M, n_keys);  // the caller sized n_keys for the fullest cell
         __syncthreads();
         if (pc.M <= 4 * WAVE) sort_candidates<D, 4>(Gs, pc, s_key);
         else if (pc.M <= 8 * WAVE) sort_candidates<D, 8>(Gs, pc, s_key);

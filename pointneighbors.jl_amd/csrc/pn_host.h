@@ -183,7 +183,10 @@ struct pn_grid {
     Buf csr_counts;
     Buf csr_status;
     Scanner csr_scan;
-    pn::DevStatus* csr_host_status = nullptr;
+    pn::DevStatus* csr_host_status = nullptr;  // pinned: of the last pn_csr_count, then of the grid at that time
+    // whether csr_host_status[1] holds the grid's status, and of which binning (BinSet::mail_seq)
+    bool csr_grid_known = false;
+    unsigned long long csr_grid_seq = 0;
     int64_t err_point = -1;
     int64_t err_cell[3] = {0, 0, 0};
     const void* err_src = nullptr;
