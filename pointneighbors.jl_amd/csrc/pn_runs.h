@@ -62,7 +62,6 @@ struct RunScale {
 
 // How the sorted positions are cut into runs.
 struct RunSplit {
-    int n;     // points of the query set, -1: read on the device
     int most;  // queries of a run, a power of two up to RUN
     int lg_parts;  // 2^lg_parts wavefronts share the runs of a window of `most` positions
     int span;  // cells of a run
@@ -502,7 +501,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_runs_count(Geom g, SetView Q, SetVi
 #pragma unroll
     for (int d = 0; d < D; ++d) box[d] = (TR)g.box[d];
     const TR r2_in = r2 - r2 * (TR)sc.cell_rel;  // up to this x distance squared cells are adjacent
-    const int n = sp.n >= 0 ? sp.n : Q.st->n_binned;
+    const int n = Q.st->n_binned;
     const int n_work = (n + sp.most - 1) / sp.most << sp.lg_parts;
     const int xcd = blockIdx.x & 7, per_xcd = nblocks >> 3;
     const int wchunk = (n_work + 7) >> 3;
@@ -694,7 +693,7 @@ __global__ __launch_bounds__(WAVE, (sizeof(TR) == 8 ? 3 : 4)) void k_runs(Geom g
 #pragma unroll
     for (int d = 0; d < D; ++d) box[d] = (TR)g.box[d];
     const TR r2_in = r2 - r2 * (TR)sc.cell_rel;  // up to this x distance squared cells are adjacent
-    const int n = sp.n >= 0 ? sp.n : Q.st->n_binned;
+    const int n = Q.st->n_binned;
     const int n_work = (n + sp.most - 1) / sp.most << sp.lg_parts;
     const int xcd = blockIdx.x & 7, per_xcd = nblocks >> 3;
     const int wchunk = (n_work + 7) >> 3;
