@@ -73,12 +73,16 @@ PACKED_LIST_ENTRIES = 12_000_000
 
 
 def _list_records(nl, ndims, code, n, rows, records=1):
-    """The workspace of a packed list call for `rows` selected rows over n points, or None."""
+    """The workspace of a packed list call for `rows` selected rows over n points, or None: the
+    direct kernels, also where the memory has no room for it."""
     import torch
     entries = nl.col_idx.numel() * rows // max(nl.n, 1)
     if entries < PACKED_LIST_ENTRIES or entries < 24 * n or (code == PN_FLOAT64 and ndims == 2):
         return None
-    return torch.empty(load().pn_list_pack_bytes(code, records * n), dtype=torch.uint8, device=nl.col_idx.device)
+    try:
+        return torch.empty(load().pn_list_pack_bytes(code, records * n), dtype=torch.uint8, device=nl.col_idx.device)
+    except torch.OutOfMemoryError:
+        return None
 
 
 class KernelFunctor:
