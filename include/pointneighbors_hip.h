@@ -293,6 +293,17 @@ int pn_set_tuning(pn_grid_t grid, const char* key, int64_t value);
  * max, in launch order), their number to *n, and clears the records. */
 int pn_grid_launch_times(pn_grid_t grid, float* ms, int64_t max, int64_t* n);
 
+/* Diagnostic, no reference counterpart: the kernel that the grid's last traversal (of a functor, or
+ * of a list count or fill) was launched with. */
+#define PN_TRAVERSAL_NONE 0         /* none yet */
+#define PN_TRAVERSAL_RUNS 1         /* runs of query points */
+#define PN_TRAVERSAL_CELLS 2        /* candidate-major cells, small chunks */
+#define PN_TRAVERSAL_CELLS_LARGE 3  /* ... large chunks */
+#define PN_TRAVERSAL_SLICES 4       /* per-query slices, small chunks */
+#define PN_TRAVERSAL_SLICES_LARGE 5 /* ... large chunks */
+#define PN_TRAVERSAL_SORTED_FILL 6  /* list fill in ascending order */
+int pn_grid_last_traversal(pn_grid_t grid, int* kernel);
+
 /* Adds U[-amplitude, amplitude] to each of the n values of x (a pure function of seed,
  * *step and the index), then increments *step on the device: a replayable per-step
  * perturbation like benchmarks/update.jl:28-49.  Enqueue only. */

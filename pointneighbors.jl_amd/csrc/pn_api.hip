@@ -340,6 +340,12 @@ int pn_grid_launch_times(pn_grid_t grid, float* ms, int64_t max, int64_t* n) {
     return PN_OK;
 }
 
+int pn_grid_last_traversal(pn_grid_t grid, int* kernel) {
+    if (!grid || !kernel) return fail(PN_ERR_ARGUMENT, "NULL pointer");
+    *kernel = grid->last_traversal;
+    return PN_OK;
+}
+
 int pn_set_tuning(pn_grid_t grid, const char* key, int64_t value) {
     if (!grid || !key) return fail(PN_ERR_ARGUMENT, "NULL pointer");
     const std::string k(key);

@@ -121,6 +121,7 @@ int pn_csr_fill(pn_grid_t grid, int queries, int64_t n_rows, const int32_t* row_
         int n_keys = 4 * pn::WAVE;
         while (n_keys < 27 * max_count) n_keys *= 2;
         const pn::FillArgs a{inv, row_ptr, col_idx, index_base};
+        g.last_traversal = PN_TRAVERSAL_SORTED_FILL;
         LaunchTimer timer(g);  // brackets the one traversal kernel launched below
         return dispatch_trav(g, [&](auto dc, auto tcv, auto trv) -> int {
             if constexpr (decltype(dc)::value == 3) {

@@ -195,6 +195,7 @@ struct pn_grid {
     int time_launches = 0;
     std::vector<hipEvent_t> timing_events;
     size_t timing_used = 0;
+    int last_traversal = PN_TRAVERSAL_NONE;
 
     ~pn_grid() {
         for (hipEvent_t e : timing_events) (void)hipEventDestroy(e);
@@ -636,6 +637,7 @@ int launch_runs(pn_grid& g, const BinSet* Q, const F& f) {
     pn::RunSplit sp;
     run_params(g, n, F::kLight, g.grid.fresh, sc, sp);
     const int nblocks = (int)std::min<int64_t>(round_up8((n + sp.most - 1) / sp.most << sp.lg_parts), g.persist_blocks);
+    g.last_traversal = PN_TRAVERSAL_RUNS;
     LaunchTimer timer(g);  // brackets the one traversal kernel launched below
     auto launch = [&](auto perc) {
         constexpr bool PER = decltype(perc)::value;
@@ -688,6 +690,7 @@ int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* 
         // per-query algorithm asked for
         using TCELL = std::conditional_t<(sizeof(TC) == 8 || sizeof(TR) == 8), double, float>;
         const bool large_h = g.chunk < 0 ? !F::kQueue : g.chunk == 1;
+        g.last_traversal = large_h ? PN_TRAVERSAL_SLICES_LARGE : PN_TRAVERSAL_SLICES;
         auto launch_h = [&](auto chunk, auto perc) {
             constexpr int CHK = decltype(chunk)::value;
             constexpr bool PER = decltype(perc)::value;
@@ -707,6 +710,7 @@ int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* 
         return PN_OK;
     }
     if (g.geom.hash) {  // a SpatialHashingCellList binned from the current coordinates
+        g.last_traversal = g.chunk != 0 ? PN_TRAVERSAL_CELLS_LARGE : PN_TRAVERSAL_CELLS;
         auto launch_hc = [&](auto gc, auto perc) {
             constexpr int GG = decltype(gc)::value;
             constexpr bool PER = decltype(perc)::value;
@@ -727,6 +731,7 @@ int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* 
     }
     if (g.algorithm == 0 || g.geom.periodic) {  // k_traverse does not handle periodic boxes
         constexpr int GG = pn::CellGroups<TC, F>::small;
+        g.last_traversal = PN_TRAVERSAL_CELLS;
         if (g.geom.periodic)
             hipLaunchKernelGGL((pn::k_cells<D, TC, TR, F, GG, true>), dim3(nblocks), dim3(pn::WAVE), 0, g.stream,
                                g.geom, Q->view(), g.grid.view(), r2, f, nblocks);
@@ -737,6 +742,7 @@ int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* 
         return PN_OK;
     }
     const bool large = g.chunk < 0 ? !F::kQueue : g.chunk == 1;
+    g.last_traversal = large ? PN_TRAVERSAL_SLICES_LARGE : PN_TRAVERSAL_SLICES;
     if (large)
         hipLaunchKernelGGL((pn::k_traverse<D, TC, TR, F, Chunk<TC, F>::large>), dim3(nblocks), dim3(pn::WAVE), 0,
                            g.stream, g.geom, Q->view(), g.grid.view(), r2, f, nblocks);

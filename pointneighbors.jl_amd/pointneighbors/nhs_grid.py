@@ -12,7 +12,7 @@ import itertools
 import numpy as np
 
 from . import _device
-from ._lib import (PN_ERR_OUT_OF_BOUNDS, PN_QUERIES_BINNED, PN_QUERIES_GRID, ArgumentError,
+from ._lib import (PN_ERR_OUT_OF_BOUNDS, PN_QUERIES_BINNED, PN_QUERIES_GRID, TRAVERSALS, ArgumentError,
                    BoundsError, PointNeighborsError, check, load)
 from .cell_lists import FullGridCellList, SpatialHashingCellList
 from .util import FLOAT64_EPS, dtype_code, floor_to_int, promote, scalar_dtype, wrap_int64
@@ -228,9 +228,10 @@ class GridNeighborhoodSearch(metaclass=_GridMeta):
 
     def set_tuning(self, key, value):
         """Autotuner knobs: "algorithm" (0: runs of queries, or candidate-major cells where
-        those are faster, 1: per-query candidate slices), "persist_blocks" (traversal workgroups, multiple of 8), "chunk" (-1 per
-        functor, 0 small, 1 large candidate chunk), "canonical_order" (1: in-cell order by
-        original index; 0: atomic order, nondeterministic inside a cell)."""
+        those are faster, 1: per-query candidate slices), "persist_blocks" (traversal
+        workgroups, multiple of 8), "chunk" (-1 per functor, 0 small, 1 large candidate chunk;
+        runs of queries have none), "canonical_order" (1: in-cell order by original index;
+        0: atomic order, nondeterministic inside a cell)."""
         self._tuning[key] = int(value)
         if self._handle is not None:
             check(load().pn_set_tuning(self._handle, key.encode(), int(value)), "set_tuning")
@@ -439,6 +440,12 @@ class GridNeighborhoodSearch(metaclass=_GridMeta):
         n = ctypes.c_int64()
         check(load().pn_grid_launch_times(self._handle, buf, max_launches, ctypes.byref(n)), "launch_times")
         return [buf[i] for i in range(min(n.value, max_launches))]
+
+    def last_traversal(self):
+        """The kernel that the last traversal was launched with: one of _lib.TRAVERSALS."""
+        k = ctypes.c_int()
+        check(load().pn_grid_last_traversal(self._handle, ctypes.byref(k)), "last_traversal")
+        return TRAVERSALS[k.value]
 
     def stats(self):
         lib = load()

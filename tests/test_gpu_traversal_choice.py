@@ -1,0 +1,74 @@
+"""Which kernel a traversal is launched with, on both sides of the lines where the choice changes.
+(That the kernels agree there is tested in test_gpu_run_rules.py and test_gpu_fill_sorted.py.)"""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+import pointneighbors as pn
+from pointneighbors import sph
+from pointneighbors._lib import PN_QUERIES_GRID, check, load
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def search(D, n, a_cell, dtype=np.float32, seed=1):
+    """A grid of n uniform points, a_cell per cell of edge 1."""
+    from test_gpu_parity import dev, make_nhs
+    pts = np.random.default_rng(seed).uniform(0.0, (n / a_cell) ** (1 / D), (n, D)).astype(dtype)
+    nhs = make_nhs(pts, dtype(1.0), pts.min(axis=0) - 3, pts.max(axis=0) + 3, cap=1000)
+    x = dev(pts)
+    pn.initialize(nhs, x, x)
+    return nhs, x
+
+
+def count(nhs, x, y):
+    pn.foreach_point_neighbor(pn.CountNeighbors(torch.zeros(x.shape[1], dtype=torch.int32, device="cuda")), x, y, nhs)
+    return nhs.last_traversal()
+
+
+def density(nhs, x, y):
+    m = torch.ones(y.shape[1], dtype=y.dtype, device="cuda")
+    rho = torch.zeros(x.shape[1], dtype=y.dtype, device="cuda")
+    pn.foreach_point_neighbor(sph.SPHDensity(rho, m, 0.5), x, y, nhs)
+    return nhs.last_traversal()
+
+
+@pytest.mark.parametrize("chunk", [-1, 0, 1])
+def test_knobs(chunk):
+    nhs, x = search(3, 5000, 10.0)
+    assert nhs.last_traversal() == "none"
+    nhs.set_tuning("chunk", chunk)
+    assert count(nhs, x, x) == "runs" and density(nhs, x, x) == "runs"
+    nhs.set_tuning("algorithm", 1)
+    assert count(nhs, x, x) == ("slices" if chunk == 0 else "slices (large chunks)")
+    assert density(nhs, x, x) == ("slices (large chunks)" if chunk == 1 else "slices")
+
+
+@pytest.mark.parametrize("n,want", [(32767, "cells"), (32768, "runs")])
+def test_2d(n, want):
+    nhs, x = search(2, n, 5.0)
+    assert density(nhs, x, x) == want and count(nhs, x, x) == "runs"
+
+
+@pytest.mark.parametrize("n_x,want", [(9999, "cells"), (10000, "runs")])
+def test_sparse_queries(n_x, want):
+    nhs, y = search(3, 80_000, 10.0)
+    x = y[:, :n_x].t().contiguous().t()
+    assert count(nhs, x, y) == want
+
+
+@pytest.mark.parametrize("D,n,a_cell,want", [(3, 100_000, 14.0, "sorted fill"), (3, 99_999, 14.0, "cells"),
+                                             (3, 100_000, 11.0, "cells"), (2, 100_000, 14.0, "cells")])
+def test_list_fill(D, n, a_cell, want):
+    nhs, x = search(D, n, a_cell)
+    vp = lambda t: ctypes.c_void_p(t.data_ptr())
+    rp = torch.empty(n + 1, dtype=torch.int32, device="cuda")
+    nnz, longest = ctypes.c_int64(), ctypes.c_int64()
+    check(load().pn_csr_count(nhs._handle, PN_QUERIES_GRID, n, vp(rp), 0, ctypes.byref(nnz), ctypes.byref(longest)))
+    assert nhs.last_traversal() == "cells"
+    col = torch.empty(nnz.value, dtype=torch.int32, device="cuda")
+    check(load().pn_csr_fill(nhs._handle, PN_QUERIES_GRID, n, vp(rp), vp(col), 0))
+    assert nhs.last_traversal() == want
