@@ -276,10 +276,11 @@ int pn_batch_create(int ndims, int coord_dtype, int radius_dtype, int cell_dtype
 
 /* Tuning knobs (the autotuner's choices).  No reference counterpart.  None changes a
  * neighbour set; "algorithm" and "chunk" change the order of floating-point sums.
- *   "algorithm"        0: runs of query points (default), 1: per-query candidate slices
+ *   "algorithm"        0: runs of query points, or candidate-major cells where those are faster
+ *                      (default), 1: per-query candidate slices
  *   "persist_blocks"   workgroups of the persistent traversal grid (multiple of 8)
- *   "chunk"            candidates per chunk of the slices and of a spatial-hash traversal:
- *                      -1 per functor, 0 small, 1 large
+ *   "chunk"            candidates per chunk of the slices and the cells (runs of query points have
+ *                      none): -1 per functor, 0 small, 1 large
  *   "canonical_order"  1: in-cell order by original index; 0: atomic order
  *   "pair_cache", "pair_cache_per_point"  accepted without effect (testing every candidate
  *                      again is faster than replaying recorded pairs)

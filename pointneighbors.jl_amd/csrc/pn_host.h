@@ -730,14 +730,22 @@ int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* 
         return PN_OK;
     }
     if (g.algorithm == 0 || g.geom.periodic) {  // k_traverse does not handle periodic boxes
-        constexpr int GG = pn::CellGroups<TC, F>::small;
-        g.last_traversal = PN_TRAVERSAL_CELLS;
-        if (g.geom.periodic)
-            hipLaunchKernelGGL((pn::k_cells<D, TC, TR, F, GG, true>), dim3(nblocks), dim3(pn::WAVE), 0, g.stream,
+        g.last_traversal = g.chunk != 0 ? PN_TRAVERSAL_CELLS_LARGE : PN_TRAVERSAL_CELLS;
+        auto launch_c = [&](auto gc, auto perc) {
+            constexpr int GG = decltype(gc)::value;
+            constexpr bool PER = decltype(perc)::value;
+            hipLaunchKernelGGL((pn::k_cells<D, TC, TR, F, GG, PER>), dim3(nblocks), dim3(pn::WAVE), 0, g.stream,
                                g.geom, Q->view(), g.grid.view(), r2, f, nblocks);
-        else
-            hipLaunchKernelGGL((pn::k_cells<D, TC, TR, F, GG, false>), dim3(nblocks), dim3(pn::WAVE), 0, g.stream,
-                               g.geom, Q->view(), g.grid.view(), r2, f, nblocks);
+        };
+        using Large = pn::IntC<pn::CellGroups<TC, F>::large>;
+        using Small = pn::IntC<pn::CellGroups<TC, F>::small>;
+        if (g.geom.periodic) {
+            if (g.chunk != 0) launch_c(Large{}, std::true_type{});
+            else launch_c(Small{}, std::true_type{});
+        } else {
+            if (g.chunk != 0) launch_c(Large{}, std::false_type{});
+            else launch_c(Small{}, std::false_type{});
+        }
         PN_CHECK_LAUNCH();
         return PN_OK;
     }
