@@ -1,9 +1,11 @@
 """Autotuner of the traversal launch and build strategy.
 
 Knobs (pn_set_tuning):
+  algorithm        traversal: 0 runs of queries, or candidate-major cells where those are
+                   faster, 1 per-query candidate slices
   persist_blocks   workgroups of the persistent traversal grid (occupancy vs tail)
-  chunk            LDS candidate chunk per wavefront: 0 small (more waves per CU),
-                   1 large (fewer chunk passes)
+  chunk            LDS candidate chunk per wavefront of the cells and the slices: 0 small
+                   (more waves per CU), 1 large (fewer chunk passes); runs have none
   canonical_order  build strategy: 1 ranks points inside a cell by original index
                    (deterministic), 0 keeps the atomic order of the histogram pass
                    (the reference ParallelUpdate's order; only with allow_nondeterministic)
@@ -52,7 +54,10 @@ def _time(step, reps, warmup):
 
 def autotune(search, step, *, space=None, reps=5, warmup=2, allow_nondeterministic=False, cache=None,
              key=None):
-    """Returns (best_params, table); applies the best parameters to `search`."""
+    """Returns (best_params, table); applies the best parameters to `search`.  Of the default space,
+    combinations that differ only in a chunk that the step's (last) traversal does not have are
+    timed once."""
+    default = space is None
     space = dict(DEFAULT_SPACE if space is None else space)
     if allow_nondeterministic and 0 not in space.get("canonical_order", []):
         space["canonical_order"] = list(space.get("canonical_order", [1])) + [0]
@@ -60,12 +65,17 @@ def autotune(search, step, *, space=None, reps=5, warmup=2, allow_nondeterminist
         space["canonical_order"] = [1]
     names = list(space)
     table = []
+    kernel = "none"
     for combo in itertools.product(*(space[k] for k in names)):
         params = dict(zip(names, combo))
+        if default and kernel == "runs" and params == dict(table[-1]["params"], chunk=params["chunk"]):
+            continue
         for k, v in params.items():
             search.set_tuning(k, v)
         ms = _time(step, reps, warmup)
         table.append({"params": params, "ms": ms})
+        if default:
+            kernel = search.last_traversal()
     best = min(table, key=lambda e: e["ms"])
     for k, v in best["params"].items():
         search.set_tuning(k, v)

@@ -14,7 +14,7 @@ import ctypes
 import numpy as np
 
 from . import _device
-from ._lib import PN_QUERIES_GRID, ArgumentError, PointNeighborsError, check, load
+from ._lib import PN_QUERIES_GRID, TRAVERSALS, ArgumentError, PointNeighborsError, check, load
 from .cell_lists import FullGridCellList
 from .util import dtype_code, promote, scalar_dtype
 
@@ -114,6 +114,12 @@ class BatchedGridNeighborhoodSearch:
         if self._handle is None:
             raise PointNeighborsError("update the batch once before tuning it")
         check(load().pn_set_tuning(self._handle, key.encode(), int(value)), "set_tuning")
+
+    def last_traversal(self):
+        """As GridNeighborhoodSearch.last_traversal."""
+        k = ctypes.c_int()
+        check(load().pn_grid_last_traversal(self._handle, ctypes.byref(k)), "last_traversal")
+        return TRAVERSALS[k.value]
 
 
 def displace_uniform(x, amplitude, seed, step):
