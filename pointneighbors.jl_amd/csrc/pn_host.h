@@ -584,7 +584,7 @@ bool runs_apply(const pn_grid& g, int64_t n) {
 }
 
 // Launch parameters of the run kernels for n query points, as far as the host knows (the kernels read
-// the number on the device: a replayed binning may have changed it).
+// the number on the device: a replayed binning may have changed it); n_sel: at most so many.
 // Runs of 32 queries do the least work; shorter ones put more wavefronts on a small cloud and end
 // sooner.  Measured at r = 2.4 spacings, F32, us with 8 / 16 / 32: density 15.6 / 18.4 / 22.5 at
 // 15,600 points, 20.5 / 19.3 / 24.1 at 32,768, 30.2 / 24.2 / 23.5 at 64,000, 160 / 105 / 80 at 512,000;
@@ -592,7 +592,7 @@ bool runs_apply(const pn_grid& g, int64_t n) {
 // are sparser than the grid's points have more candidates per run, so more work in each: they count
 // as fewer (100,000 probes among 512,000 bodies: n-body 87 / 68 / 86 us).
 // fresh: the grid was binned from the current coordinates.
-void run_params(const pn_grid& g, int64_t n, bool light, bool fresh, pn::RunScale& sc, pn::RunSplit& sp) {
+void run_params(const pn_grid& g, int64_t n, int64_t n_sel, bool light, bool fresh, pn::RunScale& sc, pn::RunSplit& sp) {
     const pn::Geom& geom = g.geom;
     const double radius = g.radius;
     sc = pn::RunScale{};
@@ -600,6 +600,7 @@ void run_params(const pn_grid& g, int64_t n, bool light, bool fresh, pn::RunScal
     (void)std::frexp(radius, &e);  // radius = m 2^e, m in [1/2, 1)
     sc.s = (float)std::ldexp(1.0, 1 - e);
     sc.rt = (float)radius * sc.s;
+    sp.n = (int)n_sel;
     const int64_t nc = g.grid.n_sel;
     const double work = n < nc ? (double)n * std::sqrt((double)n / (double)nc) : (double)n;
     sp.most = light ? (work >= 32768 ? 32 : (work >= 8192 ? 16 : 8)) : (work >= 65536 ? 32 : (work >= 24576 ? 16 : 8));
@@ -628,6 +629,9 @@ void run_params(const pn_grid& g, int64_t n, bool light, bool fresh, pn::RunScal
     if (sc.cell_rel > 0x1p-6 || !fresh) sp.span = 1;
 }
 
+// Wavefronts of a run kernel's launch: as many on each XCD as it has work items (pn::for_windows).
+int64_t run_blocks(const pn::RunSplit& sp) { return round_up8((sp.n + sp.most - 1) / sp.most) << sp.lg_parts; }
+
 template <int D, class TC, class TR, class F>
 int launch_runs(pn_grid& g, const BinSet* Q, const F& f) {
     const int64_t n = Q->stats_known ? Q->stats.n_binned : Q->n_sel;
@@ -635,8 +639,8 @@ int launch_runs(pn_grid& g, const BinSet* Q, const F& f) {
     const TR r = (TR)g.radius, r2 = r * r;
     pn::RunScale sc;
     pn::RunSplit sp;
-    run_params(g, n, F::kLight, g.grid.fresh, sc, sp);
-    const int nblocks = (int)std::min<int64_t>(round_up8((n + sp.most - 1) / sp.most << sp.lg_parts), g.persist_blocks);
+    run_params(g, n, Q->n_sel, F::kLight, g.grid.fresh, sc, sp);
+    const int nblocks = (int)std::min<int64_t>(run_blocks(sp), g.persist_blocks);
     g.last_traversal = PN_TRAVERSAL_RUNS;
     LaunchTimer timer(g);  // brackets the one traversal kernel launched below
     auto launch = [&](auto perc) {

@@ -62,6 +62,7 @@ struct RunScale {
 
 // How the sorted positions are cut into runs.
 struct RunSplit {
+    int n;     // points that the host expects; the kernels read their number on the device
     int most;  // queries of a run, a power of two up to RUN
     int lg_parts;  // 2^lg_parts wavefronts share the runs of a window of `most` positions
     int span;  // cells of a run
@@ -99,16 +100,45 @@ __device__ __forceinline__ unsigned div_magic(unsigned x, unsigned n, unsigned m
     return x - q * n >= n ? q + 1 : q;
 }
 
-// Calls fn(RunDesc) for the runs of work item w, the window of `most` (at most RUN) sorted positions
-// from (w >> lg_parts) * most: it is cut where the x-row changes, where a run would cover more than
-// `span` cells and at gaps.  The window's work items take its runs in turn.
+// Calls fn(w, part) for the work items of this workgroup: window w holds the sorted positions from
+// w * most on, part is which of its 2^lg_parts wavefronts this one is.  An XCD takes consecutive
+// windows, the last XCD its own from the last to the first.  Those are the cloud's outer layer in the
+// slowest dimension, and one that the cells cut thin has few points a row: its runs cover up to 32
+// cells and take some times as long as others, and started last they kept the chip waiting (us, all
+// ascending / as here, lattices whose last layer is thin: 512,000 points at r = 2.4 spacings count
+// 100 / 69, density 153 / 97; 1 M at 3.2 count 236 / 146, density 401 / 276, interact! 626 / 448; without
+// such a layer the same).
+// sp.n shares the windows out, so that no load waits for n, the number of points on the device (0.3 us
+// of a launch); where n is larger, the windows behind follow in turn.
+template <class Fn>
+__device__ __forceinline__ void for_windows(int n, int nblocks, const RunSplit& sp, Fn&& fn) {
+    const int n_win = (sp.n + sp.most - 1) / sp.most;
+    const int xcd = blockIdx.x & 7, chunk = (n_win + 7) >> 3;
+    const int w0 = min(n_win, xcd * chunk), nw = min(n_win, w0 + chunk) - w0;
+    for (int k = (int)(blockIdx.x >> 3);; k += nblocks >> 3) {
+        const int i = k >> sp.lg_parts, part = k & ((1 << sp.lg_parts) - 1);
+        int w;
+        if (i < nw) {
+            w = w0 + (xcd == 7 ? nw - 1 - i : i);
+        } else {
+            w = n_win + (i - nw) * 8 + xcd;
+            if ((int64_t)w * sp.most >= n) break;
+        }
+        fn(w, part);
+    }
+}
+
+// Calls fn(RunDesc) for the runs of window w that are this part's, every 2^lg_parts-th: the window of
+// `most` (at most RUN) sorted positions is cut where the x-row changes, where a run would cover more
+// than `span` cells and at gaps.
 template <int D, class Fn>
-__device__ __forceinline__ void for_runs(const Geom& g, const SetView& Q, int w, int n, const RunSplit& sp, Fn&& fn) {
+__device__ __forceinline__ void for_runs(const Geom& g, const SetView& Q, int w, int part, int n, const RunSplit& sp,
+                                         Fn&& fn) {
     const int lane = threadIdx.x;
-    const int p0 = (w >> sp.lg_parts) * sp.most, mask = (1 << sp.lg_parts) - 1;
-    int turn = w & mask;
+    const int p0 = w * sp.most, mask = (1 << sp.lg_parts) - 1;
+    int turn = part;
+    const int key_l = Q.keys[min((int64_t)p0 + lane, Q.cap - 1)];  // lanes from cnt on are not looked at
     const int cnt = min(sp.most, n - p0);
-    const int key_l = Q.keys[p0 + min(lane, cnt - 1)];
     const int step = key_l - __shfl_up(key_l, 1, WAVE);
     RunDesc rd;
     rd.n0 = g.n[0];
@@ -502,12 +532,8 @@ __global__ __launch_bounds__(WAVE, 4) void k_runs_count(Geom g, SetView Q, SetVi
     for (int d = 0; d < D; ++d) box[d] = (TR)g.box[d];
     const TR r2_in = r2 - r2 * (TR)sc.cell_rel;  // up to this x distance squared cells are adjacent
     const int n = Q.st->n_binned;
-    const int n_work = (n + sp.most - 1) / sp.most << sp.lg_parts;
-    const int xcd = blockIdx.x & 7, per_xcd = nblocks >> 3;
-    const int wchunk = (n_work + 7) >> 3;
-    const int w_end = min(n_work, (xcd + 1) * wchunk);
-    for (int w = xcd * wchunk + (int)(blockIdx.x >> 3); w < w_end; w += per_xcd) {
-        for_runs<D>(g, Q, w, n, sp, [&](const RunDesc& rd) {
+    for_windows(n, nblocks, sp, [&](int w, int part) {
+        for_runs<D>(g, Q, w, part, n, sp, [&](const RunDesc& rd) {
             const RunLanes ln(rd.nq);
             const bool qact = ln.query < rd.nq;
             const int qpos = rd.q0 + (qact ? ln.query : 0);
@@ -629,7 +655,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_runs_count(Geom g, SetView Q, SetVi
             if (ln.cols <= 8) count += __shfl_xor(count, 8, WAVE);
             if (lane < ln.cols && qact) f.write(Q.sorted_idx[qpos], Empty{}, count);
         });
-    }
+    });
 }
 
 // fn(f), with a smoothing kernel's kind as a constant (no branch per pair).
@@ -694,12 +720,8 @@ __global__ __launch_bounds__(WAVE, (sizeof(TR) == 8 ? 3 : 4)) void k_runs(Geom g
     for (int d = 0; d < D; ++d) box[d] = (TR)g.box[d];
     const TR r2_in = r2 - r2 * (TR)sc.cell_rel;  // up to this x distance squared cells are adjacent
     const int n = Q.st->n_binned;
-    const int n_work = (n + sp.most - 1) / sp.most << sp.lg_parts;
-    const int xcd = blockIdx.x & 7, per_xcd = nblocks >> 3;
-    const int wchunk = (n_work + 7) >> 3;
-    const int w_end = min(n_work, (xcd + 1) * wchunk);
-    for (int w = xcd * wchunk + (int)(blockIdx.x >> 3); w < w_end; w += per_xcd) {
-        for_runs<D>(g, Q, w, n, sp, [&](const RunDesc& rd) {
+    for_windows(n, nblocks, sp, [&](int w, int part) {
+        for_runs<D>(g, Q, w, part, n, sp, [&](const RunDesc& rd) {
             const RunLanes ln(rd.nq);
             const bool qact = ln.query < rd.nq;
             const int qpos = rd.q0 + (qact ? ln.query : 0);
@@ -831,7 +853,7 @@ __global__ __launch_bounds__(WAVE, (sizeof(TR) == 8 ? 3 : 4)) void k_runs(Geom g
             if (ln.cols <= 8) f.combine(acc, shfl_acc(acc, lane ^ 8));
             if (lane < ln.cols && qact) f.write(orig, qst, acc);
         });
-    }
+    });
 }
 
 }  // namespace pn

@@ -59,3 +59,28 @@ def test_dropped_points(n, D):
         full = torch.full((n,), UNTOUCHED, dtype=torch.int64, device="cuda")
         check(load().pn_sum_neighbor_indices(listed._handle, PN_QUERIES_GRID, ctypes.c_void_p(full.data_ptr()), 0, 0))
         assert torch.equal(sums, full)
+
+
+@pytest.mark.parametrize("n,fewer", [(700, 40), (700, 699), (40_000, 300), (40_000, 39_000)])
+def test_more_points_than_the_host_knows(n, fewer):
+    """A replay bins more points than the program's own last update did."""
+    from test_gpu_parity import dev, gpu_counts, gpu_sums, make_nhs
+    side = (n / 8.0) ** (1 / 3)
+    pts = np.random.default_rng(n).uniform(0.0, side, (n, 3)).astype(np.float32)
+    nhs, plain = (make_nhs(pts, np.float32(1.0), pts.min(axis=0) - 3, pts.max(axis=0) + 3, cap=1000) for _ in range(2))
+    x = dev(pts)
+    pn.initialize(nhs, x, x)
+    pn.initialize(plain, x, x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        pn.update(nhs, x, x, check_errors=False)
+    nhs._set_stream(x)
+    check(load().pn_grid_update(nhs._handle, ctypes.c_void_p(x.data_ptr()), n, 0, fewer, None))
+    graph.replay()
+    counts = torch.zeros(n, dtype=torch.int32, device="cuda")
+    sums = torch.zeros(n, dtype=torch.int64, device="cuda")
+    check(load().pn_count_neighbors(nhs._handle, PN_QUERIES_GRID, ctypes.c_void_p(counts.data_ptr()), 0))
+    check(load().pn_sum_neighbor_indices(nhs._handle, PN_QUERIES_GRID, ctypes.c_void_p(sums.data_ptr()), 0, 0))
+    assert np.array_equal(counts.cpu().numpy(), gpu_counts(plain, x, x))
+    assert np.array_equal(sums.cpu().numpy(), gpu_sums(plain, x, x))
