@@ -185,7 +185,7 @@ int pn_count_neighbors_noalloc(int ndims, int coord_dtype, int radius_dtype, int
     const bool runs = runs_apply<pn::CountF>(g, n);
     pn::RunScale sc;
     pn::RunSplit sp;
-    run_params(g, n, n, true, true, sc, sp);
+    run_params(g, n, n, true, sc, sp);
     const int64_t nwork = runs ? run_blocks(sp) : std::min<int64_t>(C, n);
     const int nblocks = (int)std::min<int64_t>(round_up8(nwork), int64_t(1) << 20);
     rc = dispatch_trav(g, [&](auto dc, auto tcv, auto trv) -> int {

@@ -83,6 +83,7 @@ struct DevStatus {
     // k_bin's minimum, moved to first_bad and set back to ~0 by the scan, so that the next binning
     // finds it ready without a launch of its own
     unsigned long long bad_now;
+    int moved;  // the coordinate planes were gathered again since (k_regather)
 };
 
 // Host copy of a binning's status in pinned, coherent host memory.  The scan (or k_build_small),
@@ -131,6 +132,7 @@ static __global__ void k_reset_status(DevStatus* st) {
     st->n_binned = 0;
     st->n_ordered = 0;
     st->bad_now = ~0ull;
+    st->moved = 0;
 }
 
 static __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
@@ -375,6 +377,7 @@ __device__ __forceinline__ void publish_status(DevStatus* st, StatusMailbox* mb,
     s.n_binned = (int)(uint32_t)(sum & 0xffffffffull);
     s.n_ordered = 0;
     s.bad_now = ~0ull;
+    s.moved = 0;
     *st = s;
     if (mb) {
         mb->status = s;
@@ -819,10 +822,11 @@ static __global__ __launch_bounds__(ORDER_THREADS) void k_order_work(const int32
 
 // Re-gathers the sorted coordinate planes from y (update-free coordinate refresh).
 template <int D, class TC>
-__global__ __launch_bounds__(256) void k_regather(const int32_t* __restrict__ sorted_idx, const DevStatus* st,
+__global__ __launch_bounds__(256) void k_regather(const int32_t* __restrict__ sorted_idx, DevStatus* st,
                                                   const TC* __restrict__ y, TC* __restrict__ coords,
                                                   int64_t cap) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k == 0) st->moved = 1;
     if (k >= st->n_binned) return;
     const int64_t p = sorted_idx[k];
 #pragma unroll

@@ -591,8 +591,7 @@ bool runs_apply(const pn_grid& g, int64_t n) {
 // count 9.6 / 9.8 / 10.8 at 4096, 14.7 / 12.2 / 12.2 at 32,768, 104 / 62 / 43 at 512,000.  Queries that
 // are sparser than the grid's points have more candidates per run, so more work in each: they count
 // as fewer (100,000 probes among 512,000 bodies: n-body 87 / 68 / 86 us).
-// fresh: the grid was binned from the current coordinates.
-void run_params(const pn_grid& g, int64_t n, int64_t n_sel, bool light, bool fresh, pn::RunScale& sc, pn::RunSplit& sp) {
+void run_params(const pn_grid& g, int64_t n, int64_t n_sel, bool light, pn::RunScale& sc, pn::RunSplit& sp) {
     const pn::Geom& geom = g.geom;
     const double radius = g.radius;
     sc = pn::RunScale{};
@@ -620,13 +619,13 @@ void run_params(const pn_grid& g, int64_t n, int64_t n_sel, bool light, bool fre
         sc.per_mg = (float)(len * sc.s * sc.rt * 0x1p-19);
     }
     // (x - min) / cell size has a relative error below 2 u, so a pair two cells apart is at least
-    // r (1 - 4 u n) away; twice that for d^2, and its own rounding.  Where that bound is useless, or
-    // the cells are those of earlier coordinates, runs are single cells.
+    // r (1 - 4 u n) away; twice that for d^2, and its own rounding.  Where that bound is useless, runs
+    // are single cells.
     sp.cell64 = g.tcell == PN_FLOAT64;
     int64_t n0 = geom.n[0];
     for (const pn::GeomEntry& e : g.host_table) n0 = std::max<int64_t>(n0, e.n[0]);
     sc.cell_rel = (double)(n0 + 1) * (sp.cell64 ? 0x1p-49 : 0x1p-20) + (g.tr == PN_FLOAT64 ? 0x1p-48 : 0x1p-20);
-    if (sc.cell_rel > 0x1p-6 || !fresh) sp.span = 1;
+    if (sc.cell_rel > 0x1p-6) sp.span = 1;
 }
 
 // Wavefronts of a run kernel's launch: as many on each XCD as it has work items (pn::for_windows).
@@ -639,7 +638,7 @@ int launch_runs(pn_grid& g, const BinSet* Q, const F& f) {
     const TR r = (TR)g.radius, r2 = r * r;
     pn::RunScale sc;
     pn::RunSplit sp;
-    run_params(g, n, Q->n_sel, F::kLight, g.grid.fresh, sc, sp);
+    run_params(g, n, Q->n_sel, F::kLight, sc, sp);
     const int nblocks = (int)std::min<int64_t>(run_blocks(sp), g.persist_blocks);
     g.last_traversal = PN_TRAVERSAL_RUNS;
     LaunchTimer timer(g);  // brackets the one traversal kernel launched below

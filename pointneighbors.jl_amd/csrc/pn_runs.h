@@ -22,7 +22,8 @@
 // They are further away than r but for the rounding of the cell arithmetic, where the reference
 // does not look at them: a pair that close to r is accepted only if its cells are adjacent.  After
 // coordinates moved without a new binning a run is one cell, so that the cells of the binning
-// decide, as in the reference.
+// decide, as in the reference.  The device says so (DevStatus::moved): a captured traversal may be
+// replayed over coordinates that moved since its capture.
 // Points for which the estimate cannot be trusted (a query outside its cell after an in-place
 // move, a candidate whose other image in a periodic box may be as near) are kept as "maybe" for every pair.
 //
@@ -65,7 +66,7 @@ struct RunSplit {
     int n;     // points that the host expects; the kernels read their number on the device
     int most;  // queries of a run, a power of two up to RUN
     int lg_parts;  // 2^lg_parts wavefronts share the runs of a window of `most` positions
-    int span;  // cells of a run
+    int span;  // cells of a run (one where the coordinates moved since the binning)
     unsigned magic0, magic1;  // floor((2^32 - 1) / cells) in x and y (no batch table)
     int cell64;  // cells are computed in Float64
 };
@@ -532,6 +533,7 @@ __global__ __launch_bounds__(WAVE, 4) void k_runs_count(Geom g, SetView Q, SetVi
     for (int d = 0; d < D; ++d) box[d] = (TR)g.box[d];
     const TR r2_in = r2 - r2 * (TR)sc.cell_rel;  // up to this x distance squared cells are adjacent
     const int n = Q.st->n_binned;
+    if (Gs.st->moved) sp.span = 1;
     for_windows(n, nblocks, sp, [&](int w, int part) {
         for_runs<D>(g, Q, w, part, n, sp, [&](const RunDesc& rd) {
             const RunLanes ln(rd.nq);
@@ -720,6 +722,7 @@ __global__ __launch_bounds__(WAVE, (sizeof(TR) == 8 ? 3 : 4)) void k_runs(Geom g
     for (int d = 0; d < D; ++d) box[d] = (TR)g.box[d];
     const TR r2_in = r2 - r2 * (TR)sc.cell_rel;  // up to this x distance squared cells are adjacent
     const int n = Q.st->n_binned;
+    if (Gs.st->moved) sp.span = 1;
     for_windows(n, nblocks, sp, [&](int w, int part) {
         for_runs<D>(g, Q, w, part, n, sp, [&](const RunDesc& rd) {
             const RunLanes ln(rd.nq);
