@@ -645,6 +645,11 @@ static __global__ __launch_bounds__(BUILD_THREADS) void k_scan_one(int32_t* __re
 constexpr int BUILD_ITEMS = 4;
 constexpr int BUILD_SMALL_POINTS = BUILD_THREADS * BUILD_ITEMS;
 constexpr int BUILD_SMALL_CELLS = 11 * 1024;  // 64 KB of LDS
+// Ranking every point among those of its cell takes a compute unit too long where cells are crowded.
+// From a fullest cell of this many points on, the selection is placed in its order, 64 points at a
+// time (4096 points, 30 / 250 / 1000 a cell: ranked 22 / 86 / 291 us, placed in order 22 us from 64 on,
+// 23 / 19; the kernels of larger clouds 23 / 46 / 109).
+constexpr int BUILD_CROWDED = 64;
 
 template <int D, class TC, class TCELL>
 __global__ __launch_bounds__(BUILD_THREADS) void k_build_small(Geom g, const TC* __restrict__ y, int64_t sel_first,
@@ -661,9 +666,13 @@ __global__ __launch_bounds__(BUILD_THREADS) void k_build_small(Geom g, const TC*
     __shared__ unsigned long long sh[BUILD_THREADS / WAVE];
     __shared__ int sh_max[BUILD_THREADS / WAVE];
     __shared__ int s_bad;
+    __shared__ int s_descends;  // the selection is not in the order of the points
     const int C = g.ncells;
     for (int c = threadIdx.x; c < C; c += BUILD_THREADS) s_cell[c] = 0;
-    if (threadIdx.x == 0) s_bad = INT32_MAX;
+    if (threadIdx.x == 0) {
+        s_bad = INT32_MAX;
+        s_descends = 0;
+    }
     __syncthreads();
     int key[BUILD_ITEMS], slot[BUILD_ITEMS];
     int32_t p[BUILD_ITEMS];
@@ -673,6 +682,7 @@ __global__ __launch_bounds__(BUILD_THREADS) void k_build_small(Geom g, const TC*
         key[i] = -1;
         if (a < n_sel) {
             p[i] = (int32_t)sel_point(a, sel_first, sel_list);
+            if (sel_list && a > 0 && sel_list[a - 1] > p[i]) s_descends = 1;
             bool ok;
             const int k = point_key<D, TC, TCELL>(g, y, p[i], ok);
             if (ok) {
@@ -698,31 +708,62 @@ __global__ __launch_bounds__(BUILD_THREADS) void k_build_small(Geom g, const TC*
                        max_count, sum);
     }
     __syncthreads();
-#pragma unroll
-    for (int i = 0; i < BUILD_ITEMS; ++i)
-        if (key[i] >= 0) s_perm[s_cell[key[i]] + slot[i]] = (int)threadIdx.x + i * BUILD_THREADS;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < BUILD_ITEMS; ++i) {
-        if (key[i] < 0) continue;
-        const int a = (int)threadIdx.x + i * BUILD_THREADS, b = s_cell[key[i]], e = s_cell[key[i] + 1];
-        int pos = b + slot[i];
-        if (canonical && e - b <= CANON_RANK_LIMIT) {
-            pos = b;
-            for (int q = b; q < e; ++q) {
-                const int aq = s_perm[q];
-                if (!sel_list) {
-                    pos += aq < a;
-                } else {
-                    const int32_t pq = sel_list[aq];
-                    pos += (pq < p[i]) || (pq == p[i] && aq < a);
-                }
-            }
-        }
+    auto place = [&](int i, int pos) {
         sorted_idx[pos] = p[i];
         sorted_keys[pos] = key[i];
 #pragma unroll
         for (int d = 0; d < D; ++d) coords[(int64_t)d * cap + pos] = y[(int64_t)D * p[i] + d];
+    };
+    if (canonical && max_count >= BUILD_CROWDED && !s_descends) {  // the same for the whole workgroup
+#pragma unroll
+        for (int i = 0; i < BUILD_ITEMS; ++i) {
+            // among the wavefront's points: those of its cell, and those of them before it
+            int before = 0, n_same = 0;
+            for (unsigned long long left = __ballot(key[i] >= 0); left;) {
+                const int k = __builtin_amdgcn_readlane(key[i], __builtin_ctzll(left));
+                const unsigned long long same = __ballot(key[i] == k);
+                if (key[i] == k) {
+                    before = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(same >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((unsigned)same, 0));
+                    n_same = __popcll(same);
+                }
+                left &= ~same;
+            }
+            // the wavefronts in turn: s_cell[c] is the next free slot of cell c
+            for (int t = 0; t < BUILD_THREADS / WAVE; ++t) {
+                if (i * BUILD_THREADS + t * WAVE >= n_sel) break;
+                if ((int)threadIdx.x / WAVE == t && key[i] >= 0) {
+                    const int next = s_cell[key[i]];
+                    if (before == 0) s_cell[key[i]] = next + n_same;
+                    place(i, next + before);
+                }
+                __syncthreads();
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < BUILD_ITEMS; ++i)
+            if (key[i] >= 0) s_perm[s_cell[key[i]] + slot[i]] = (int)threadIdx.x + i * BUILD_THREADS;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < BUILD_ITEMS; ++i) {
+            if (key[i] < 0) continue;
+            const int a = (int)threadIdx.x + i * BUILD_THREADS, b = s_cell[key[i]], e = s_cell[key[i] + 1];
+            int pos = b + slot[i];
+            if (canonical && e - b <= CANON_RANK_LIMIT) {
+                pos = b;
+                for (int q = b; q < e; ++q) {
+                    const int aq = s_perm[q];
+                    if (!sel_list) {
+                        pos += aq < a;
+                    } else {
+                        const int32_t pq = sel_list[aq];
+                        pos += (pq < p[i]) || (pq == p[i] && aq < a);
+                    }
+                }
+            }
+            place(i, pos);
+        }
     }
 }
 
