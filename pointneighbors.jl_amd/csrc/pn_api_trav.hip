@@ -30,13 +30,18 @@ static bool fill_sorted_possible(const pn_grid& g, const BinSet& Q) {
     return g.grid.n_sel >= 100000 && Q.n_sel >= g.grid.n_sel;
 }
 
-// Whether it makes them, st being the grid's status: its fullest cell bounds a cell's candidates by
-// what the kernel sorts in registers.  It shares a cell's sorted candidates among the cell's queries,
-// so it needs many of them: from 12 points a cell on (us, a million points F32: 7.5 a cell 294 / 315,
-// 10 a cell 310 / 347; 216,000 points with 14 a cell 120 / 104; 2D with 16 a cell 196 / 203).
+// Whether it makes them, st being the grid's status with n_ordered what k_list_counts found: its fullest
+// cell bounds a cell's candidates by what the kernel sorts in registers.  It shares a cell's sorted
+// candidates among the cell's queries, so it needs many of them: from 14 points a cell on (us, a million
+// points F32: 7.5 a cell 294 / 315, 10 a cell 310 / 347; 216,000 points with 14 a cell 120 / 104; whole
+// builds 500,000 points with 12.5 a cell 286 / 305, F64 360 / 356, 16 a cell 376 / 328, 462 / 391; 2D with
+// 16 a cell 196 / 203).  It gathers the candidates in the order of the original indices, which has to
+// be near the order of the cells: more than four in ten of the points follow each other in both (a
+// lattice at 2.4 spacings six; whole builds 500,000 points in no order 16 a cell 415 / 438, F64 503 / 614,
+// 30 a cell 567 / 694, 734 / 1036).
 static bool fill_sorted_applies(const pn::DevStatus& st) {
-    if (st.n_binned < 100000 || st.n_binned / 12 < st.n_nonempty) return false;
-    return 27 * (int64_t)st.max_count <= pn::FILL_CAP;
+    if (st.n_binned < 100000 || st.n_binned / 14 < st.n_nonempty) return false;
+    return 27 * (int64_t)st.max_count <= pn::FILL_CAP && 10 * st.n_ordered > 4 * pn::FILL_SAMPLES;
 }
 
 // Whether work is being captured on the stream (or may be: an implicit capture refuses the query).
@@ -62,29 +67,36 @@ int pn_csr_count(pn_grid_t grid, int queries, int64_t n_rows, int32_t* row_ptr, 
     // the fill keeps the positions of the grid's points there once the counts are summed
     const int64_t n_counts = std::max(n_rows, std::max<int64_t>(g.grid.n_src, 1));
     if ((rc = g.csr_counts.ensure((size_t)n_counts * 4, g.stream))) return rc;
-    if ((rc = g.csr_status.ensure(sizeof(pn::DevStatus), g.stream))) return rc;
+    if ((rc = g.csr_status.ensure(2 * sizeof(pn::DevStatus), g.stream))) return rc;
     if (!g.csr_host_status)
         PN_HIP(hipHostMalloc((void**)&g.csr_host_status, 2 * sizeof(pn::DevStatus), hipHostMallocDefault));
     auto* st = g.csr_status.as<pn::DevStatus>();
-    hipLaunchKernelGGL(pn::k_reset_status, dim3(1), dim3(1), 0, g.stream, st);
-    PN_CHECK_LAUNCH();
-    hipLaunchKernelGGL(pn::k_fill_i32, dim3(blocks_for(std::min<int64_t>(n_rows, 1 << 20), 256)), dim3(256), 0,
-                       g.stream, g.csr_counts.as<int32_t>(), n_rows, 0);
-    PN_CHECK_LAUNCH();
-    pn::CountF f;
-    f.out = g.csr_counts.as<int32_t>();
-    f.accumulate = 0;
-    // lists are mostly made of undeformed lattices, whose ties the cell kernel counts faster
-    if ((rc = launch_traverse(g, queries, f, false))) return rc;
-    if ((rc = g.csr_scan.run(g.csr_counts.as<int32_t>(), n_rows, row_ptr, nullptr, st, g.stream))) return rc;
-    PN_HIP(hipMemcpyAsync(g.csr_host_status, st, sizeof(pn::DevStatus), hipMemcpyDeviceToHost, g.stream));
     // the grid's own status from the device: the host's copy is that of an earlier binning where a
     // captured one has been replayed
     g.csr_grid_known = fill_sorted_possible(g, *Q);
     g.csr_grid_seq = g.grid.mail_seq;
-    if (g.csr_grid_known)
-        PN_HIP(hipMemcpyAsync(g.csr_host_status + 1, g.grid.status.p, sizeof(pn::DevStatus), hipMemcpyDeviceToHost,
-                              g.stream));
+    const dim3 fill_blocks(blocks_for(std::min<int64_t>(n_rows, 1 << 20), 256));
+    if (g.csr_grid_known) {  // fewer rows than samples (points selected repeatedly) count as no order
+        hipLaunchKernelGGL(pn::k_list_status, dim3(1), dim3(1), 0, g.stream, g.grid.status.as<pn::DevStatus>(), st);
+        PN_CHECK_LAUNCH();
+        hipLaunchKernelGGL(pn::k_list_counts, fill_blocks, dim3(256), 0, g.stream, g.csr_counts.as<int32_t>(), n_rows,
+                           g.grid.sorted_idx.as<int32_t>(), st);
+    } else {
+        hipLaunchKernelGGL(pn::k_reset_status, dim3(1), dim3(1), 0, g.stream, st);
+        PN_CHECK_LAUNCH();
+        hipLaunchKernelGGL(pn::k_fill_i32, fill_blocks, dim3(256), 0, g.stream, g.csr_counts.as<int32_t>(), n_rows, 0);
+    }
+    PN_CHECK_LAUNCH();
+    pn::CountF f;
+    f.out = g.csr_counts.as<int32_t>();
+    f.accumulate = 0;
+    // lists are mostly made of undeformed lattices, whose ties the cell kernel counts faster (128^3 at
+    // r = 3 spacings F32 267 us, runs 400); other clouds' counts lose by it (1 M points at 2.4 spacings
+    // 116 us, runs 90)
+    if ((rc = launch_traverse(g, queries, f, false))) return rc;
+    if ((rc = g.csr_scan.run(g.csr_counts.as<int32_t>(), n_rows, row_ptr, nullptr, st, g.stream))) return rc;
+    PN_HIP(hipMemcpyAsync(g.csr_host_status, st, (g.csr_grid_known ? 2 : 1) * sizeof(pn::DevStatus),
+                          hipMemcpyDeviceToHost, g.stream));
     PN_HIP(hipStreamSynchronize(g.stream));
     const pn::DevStatus hs = *g.csr_host_status;
     if (nnz) *nnz = (int64_t)hs.total64;

@@ -79,7 +79,7 @@ struct DevStatus {
     int max_count;                 // largest cell population
     int n_nonempty;                // number of non-empty cells
     int n_binned;                  // number of binned points (low 32 bits of the sum)
-    int n_ordered;                 // work items appended by k_order_work
+    int n_ordered;                 // work items appended by k_order_work; k_list_counts
     // k_bin's minimum, moved to first_bad and set back to ~0 by the scan, so that the next binning
     // finds it ready without a launch of its own
     unsigned long long bad_now;

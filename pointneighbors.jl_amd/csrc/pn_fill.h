@@ -29,6 +29,39 @@ static __global__ __launch_bounds__(256) void k_invert(const int32_t* __restrict
     for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) inv[sorted_idx[p]] = p;
 }
 
+// Status of a list count: st[0] as k_reset_status leaves it; st[1] the grid's own, with n_ordered for
+// k_list_counts.
+static __global__ void k_list_status(const DevStatus* __restrict__ grid_st, DevStatus* __restrict__ st) {
+    DevStatus s = {};
+    s.first_bad = s.bad_now = ~0ull;
+    st[0] = s;
+    s = *grid_st;
+    s.n_ordered = 0;
+    st[1] = s;
+}
+
+// Clears the counts of a list count's rows and counts, among FILL_SAMPLES pairs of neighbouring sorted
+// positions spread over the grid's points, those whose original indices differ by two at most (in the
+// same launch, which it does not lengthen; one of its own took 7 us).
+constexpr int FILL_SAMPLES = 4096;
+static __global__ __launch_bounds__(256) void k_list_counts(int32_t* __restrict__ counts, int64_t n,
+                                                            const int32_t* __restrict__ sorted_idx,
+                                                            DevStatus* __restrict__ st) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < FILL_SAMPLES) {  // whole wavefronts
+        const int n_binned = st[1].n_binned;
+        bool near = false;
+        if (n_binned >= 2) {
+            const int p = (int)(t * (n_binned - 1) / FILL_SAMPLES);
+            const int64_t step = (int64_t)sorted_idx[p + 1] - sorted_idx[p];
+            near = step >= -2 && step <= 2;
+        }
+        const int in_wave = __popcll(__ballot(near));
+        if ((threadIdx.x & (WAVE - 1)) == 0) atomicAdd(&st[1].n_ordered, in_wave);
+    }
+    for (int64_t i = t; i < n; i += (int64_t)gridDim.x * blockDim.x) counts[i] = 0;
+}
+
 __device__ __forceinline__ float lane_value(float v, int l) {
     return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(v), l));
 }

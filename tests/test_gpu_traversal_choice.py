@@ -60,10 +60,18 @@ def test_sparse_queries(n_x, want):
     assert count(nhs, x, y) == want
 
 
-@pytest.mark.parametrize("D,n,a_cell,want", [(3, 100_000, 14.0, "sorted fill"), (3, 99_999, 14.0, "cells"),
-                                             (3, 100_000, 11.0, "cells"), (2, 100_000, 14.0, "cells")])
-def test_list_fill(D, n, a_cell, want):
+@pytest.mark.parametrize("D,n,a_cell,order,want", [(3, 100_000, 16.0, "cells", "sorted fill"),
+                                                   (3, 99_999, 16.0, "cells", "cells"),
+                                                   (3, 100_000, 12.5, "cells", "cells"),
+                                                   (2, 100_000, 16.0, "cells", "cells"),
+                                                   (3, 100_000, 16.0, "none", "cells")])
+def test_list_fill(D, n, a_cell, order, want):
     nhs, x = search(D, n, a_cell)
+    if order == "cells":
+        sorted_idx = torch.empty(n, dtype=torch.int32, device="cuda")
+        check(load().pn_grid_copy_cells(nhs._handle, None, ctypes.c_void_p(sorted_idx.data_ptr())))
+        x = x[:, sorted_idx.long()].t().contiguous().t()
+        pn.initialize(nhs, x, x)
     vp = lambda t: ctypes.c_void_p(t.data_ptr())
     rp = torch.empty(n + 1, dtype=torch.int32, device="cuda")
     nnz, longest = ctypes.c_int64(), ctypes.c_int64()
@@ -72,3 +80,15 @@ def test_list_fill(D, n, a_cell, want):
     col = torch.empty(nnz.value, dtype=torch.int32, device="cuda")
     check(load().pn_csr_fill(nhs._handle, PN_QUERIES_GRID, n, vp(rp), vp(col), 0))
     assert nhs.last_traversal() == want
+
+
+def test_full_rows_in_an_empty_domain():
+    """Points one to a cell on a plane of a wide domain: rows of cells are full, runs are long."""
+    from test_gpu_parity import dev, make_nhs
+    rng = np.random.default_rng(2)
+    pts = np.zeros((320 * 320, 3), np.float32)
+    pts[:, :2] = np.stack(np.meshgrid(*[np.arange(320)] * 2), -1).reshape(-1, 2) + rng.uniform(0.1, 0.9, (320 * 320, 2))
+    nhs = make_nhs(pts, np.float32(1.0), np.full(3, -50.0, np.float32), np.full(3, 370.0, np.float32), cap=1000)
+    x = dev(pts)
+    pn.initialize(nhs, x, x)
+    assert count(nhs, x, x) == "runs" and density(nhs, x, x) == "runs"
