@@ -182,10 +182,10 @@ int pn_count_neighbors_noalloc(int ndims, int coord_dtype, int radius_dtype, int
     pn::CountF f;
     f.out = counts;
     f.accumulate = 0;
-    const bool runs = runs_apply<pn::CountF>(g, n);
+    const bool runs = runs_apply<pn::CountF>(g, n, CloudCells());
     pn::RunScale sc;
     pn::RunSplit sp;
-    run_params(g, n, n, true, sc, sp);
+    run_params(g, n, CloudCells(), n, true, sc, sp);
     const int64_t nwork = runs ? run_blocks(sp) : std::min<int64_t>(C, n);
     const int nblocks = (int)std::min<int64_t>(round_up8(nwork), int64_t(1) << 20);
     rc = dispatch_trav(g, [&](auto dc, auto tcv, auto trv) -> int {

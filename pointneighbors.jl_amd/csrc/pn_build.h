@@ -84,6 +84,7 @@ struct DevStatus {
     // finds it ready without a launch of its own
     unsigned long long bad_now;
     int moved;  // the coordinate planes were gathered again since (k_regather)
+    int n_octets;  // aligned groups of eight cells (in x, but for the ends of rows) that hold points; 0: not counted
 };
 
 // Host copy of a binning's status in pinned, coherent host memory.  The scan (or k_build_small),
@@ -133,6 +134,7 @@ static __global__ void k_reset_status(DevStatus* st) {
     st->n_ordered = 0;
     st->bad_now = ~0ull;
     st->moved = 0;
+    st->n_octets = 0;
 }
 
 static __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
@@ -349,26 +351,34 @@ static __global__ __launch_bounds__(SCAN_THREADS) void k_scan_reduce(const int32
     }
     unsigned long long total;
     block_excl_scan(s, sh, total);
+    static_assert(SCAN_ITEMS == 8, "a thread's cells are an octet");
+    const int octets = __popcll(__ballot(s != 0));
     // block max of the populations; block sums and maxima go to k_scan_top (no same-address
     // atomics: with millions of cells or buckets they serialised the pass)
-    __shared__ int shm[SCAN_THREADS / WAVE];
+    __shared__ int shm[SCAN_THREADS / WAVE], sho[SCAN_THREADS / WAVE];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o, WAVE));
-    if ((threadIdx.x & (WAVE - 1)) == 0) shm[threadIdx.x >> 6] = mx;
+    if ((threadIdx.x & (WAVE - 1)) == 0) {
+        shm[threadIdx.x >> 6] = mx;
+        sho[threadIdx.x >> 6] = octets;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-        int m = shm[0];
+        int m = shm[0], oct = sho[0];
 #pragma unroll
-        for (int i = 1; i < SCAN_THREADS / WAVE; ++i) m = max(m, shm[i]);
+        for (int i = 1; i < SCAN_THREADS / WAVE; ++i) {
+            m = max(m, shm[i]);
+            oct += sho[i];
+        }
         block_sums[blockIdx.x] = total;
-        block_sums[gridDim.x + blockIdx.x] = (unsigned long long)(uint32_t)m;
+        block_sums[gridDim.x + blockIdx.x] = (unsigned long long)(uint32_t)m | (unsigned long long)oct << 32;
     }
 }
 
 // The status of a binning whose packed counts sum to `sum`; in pinned host memory too when mb.
 __device__ __forceinline__ void publish_status(DevStatus* st, StatusMailbox* mb, unsigned long long seq,
                                                unsigned long long bad, unsigned long long total64, int max_count,
-                                               unsigned long long sum) {
+                                               unsigned long long sum, int n_octets = 0) {
     DevStatus s;
     s.first_bad = bad;
     s.total64 = total64;
@@ -378,6 +388,7 @@ __device__ __forceinline__ void publish_status(DevStatus* st, StatusMailbox* mb,
     s.n_ordered = 0;
     s.bad_now = ~0ull;
     s.moved = 0;
+    s.n_octets = n_octets;
     *st = s;
     if (mb) {
         mb->status = s;
@@ -386,23 +397,25 @@ __device__ __forceinline__ void publish_status(DevStatus* st, StatusMailbox* mb,
 }
 
 // Single workgroup: exclusive scan of the block sums (block_sums[0, nblocks)), writes the
-// totals, the 64-bit sum of all counts and the largest count (block maxima at
-// block_sums[nblocks, 2 nblocks)).
+// totals, the 64-bit sum of all counts, the largest count and the number of octets (block maxima and
+// octets at block_sums[nblocks, 2 nblocks)).
 static __global__ __launch_bounds__(SCAN_THREADS) void k_scan_top(unsigned long long* __restrict__ block_sums,
                                                            int64_t nblocks, int32_t* __restrict__ start,
                                                            int64_t C, DevStatus* st, StatusMailbox* mb,
                                                            unsigned long long seq) {
     __shared__ unsigned long long sh[SCAN_THREADS / WAVE];
     __shared__ unsigned long long sh_sum[SCAN_THREADS / WAVE];
-    __shared__ int sh_max[SCAN_THREADS / WAVE];
+    __shared__ int sh_max[SCAN_THREADS / WAVE], sh_oct[SCAN_THREADS / WAVE];
     unsigned long long carry = 0, sum64 = 0;
-    int mx = 0;
+    int mx = 0, oct = 0;
     for (int64_t b0 = 0; b0 < nblocks; b0 += SCAN_THREADS) {
         int64_t b = b0 + threadIdx.x;
         unsigned long long v = b < nblocks ? block_sums[b] : 0ull;
         if (b < nblocks) {
             sum64 += v & 0xffffffffull;
-            mx = max(mx, (int)(uint32_t)block_sums[nblocks + b]);
+            const unsigned long long mo = block_sums[nblocks + b];
+            mx = max(mx, (int)(uint32_t)mo);
+            oct += (int)(uint32_t)(mo >> 32);
         }
         unsigned long long total;
         unsigned long long ex = block_excl_scan(v, sh, total);
@@ -413,22 +426,25 @@ static __global__ __launch_bounds__(SCAN_THREADS) void k_scan_top(unsigned long 
     for (int o = 32; o > 0; o >>= 1) {
         sum64 += __shfl_xor(sum64, o, WAVE);
         mx = max(mx, __shfl_xor(mx, o, WAVE));
+        oct += __shfl_xor(oct, o, WAVE);
     }
     if ((threadIdx.x & (WAVE - 1)) == 0) {
         sh_sum[threadIdx.x >> 6] = sum64;
         sh_max[threadIdx.x >> 6] = mx;
+        sh_oct[threadIdx.x >> 6] = oct;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         unsigned long long tot = 0;
-        int m = 0;
+        int m = 0, n_octets = 0;
 #pragma unroll
         for (int i = 0; i < SCAN_THREADS / WAVE; ++i) {
             tot += sh_sum[i];
             m = max(m, sh_max[i]);
+            n_octets += sh_oct[i];
         }
         start[C] = (int32_t)(uint32_t)(carry & 0xffffffffull);
-        publish_status(st, mb, seq, st->bad_now, tot, m, carry);  // bad_now: of k_bin, an earlier kernel
+        publish_status(st, mb, seq, st->bad_now, tot, m, carry, n_octets);  // bad_now: of k_bin, an earlier kernel
     }
 }
 

@@ -555,6 +555,19 @@ int check_queries(pn_grid& g, int queries, const BinSet*& Q) {
     return PN_OK;
 }
 
+// What the host knows of the cells of n points: whether they hold fewer than two on average, and how
+// full the surroundings in x of a filled cell are (filled cells per octet that has any: 1 to 8).
+struct CloudCells {
+    double per_cell = 0.0;  // points per filled cell, 0: not known
+    double in_octet = 0.0;  // 0: not known, or fuller cells
+    CloudCells() = default;
+    explicit CloudCells(const BinSet& s) {
+        if (!s.stats_known || s.stats.n_nonempty <= 0) return;
+        per_cell = (double)s.stats.n_binned / (double)s.stats.n_nonempty;
+        if (per_cell < 2.0 && s.stats.n_octets > 0) in_octet = (double)s.stats.n_nonempty / (double)s.stats.n_octets;
+    }
+};
+
 // Whether the run kernels (pn_runs.h) take a traversal of n query points: they need a cell per
 // sorted position (a FullGridCellList), lengths that Float32 holds with room for their squares, and
 // planes that a 32-bit byte offset reaches.  They are faster than the cell kernel (k_cells) over the
@@ -563,19 +576,40 @@ int check_queries(pn_grid& g, int queries, const BinSet*& Q) {
 // 24.5 -> 13) but for
 //   * queries that are sparse among the grid's points, whose runs are single points and take a
 //     wavefront's runs one after another (cells / runs, us, 512,000 points: n-body 1000 probes
-//     12 / 66, 30,000 41 / 55, 60,000 55 / 57, 120,000 72 / 61; count 21 / 41, 31 / 39, 38 / 41,
-//     44 / 46; 29,791 points: n-body 2000 probes 21 / 40, 8000 32 / 30): from one query for eight points on;
-//   * 2D pair functors over small clouds, whose cells have few candidates (density, r = 2.3 and 2.8
-//     spacings: 4200 points 7.2 / 8.1 and 7.7 / 8.5, 19,200 points 8.2 / 12.2 and 8.4 / 11, 90,000
-//     points 15.7 / 13.5 and 14.1 / 17): below 32,768 points;
-//   * counting an undeformed lattice whose search radius is a lattice distance (128^3, r = 3
-//     spacings: 305 -> 400 us, a quarter of the neighbours are ties): the list builder counts by cells.
+//     12 / 66, 30,000 41 / 55; whole calls at r = 3 spacings: count of 64,000 63 / 65, 80,000 67 / 71,
+//     120,000 76 / 69, n-body 90 / 94, 97 / 99, 114 / 106): from one query for six points on;
+//   * clouds of single points with empty cells around them, for the same reason (uniform points, whole
+//     calls, us; .02 and .1 points a cell, which are 1.07 and 1.38 filled cells in an octet: count of
+//     100,000 points 47 / 61 and 46 / 38, 500,000 186 / 267 and 175 / 135, density 60 / 75 and 55 / 47,
+//     295 / 314 and 278 / 163; 2D 37 / 62 and 37 / 36, 162 / 297 and 148 / 138; 20,000 points in 3D:
+//     count 23 / 19 and 23 / 15, density 16 / 25 and 16 / 20; 2000 points: runs);
+//   * 2D pair functors over small clouds and fuller cells: a run has the candidates of three rows over
+//     its own cells and two more, and 32 queries are few of those cells (whole calls, F32 and F64
+//     TrixiParticles interact!, r = 2 / 2.4 / 2.8 / 3.2 spacings, which are 4 to 10 points a cell; 36,100
+//     points: F64 17 / 20 at 2.4, 19 / 23 at 3.2; 57,600: F32 16.9 / 15.7, 15.8 / 16.0, 15.7 / 16.6, 17.7 / 19.1;
+//     90,000: 23 / 16, 21 / 19, 20 / 19, 21 / 22; 176,400: 39 / 21, 34 / 26, 32 / 28, 33 / 33, F64 at 3.2 55 / 58;
+//     360,000: 76 / 32, 65 / 41, 58 / 43, 59 / 52).  In a periodic box the cell kernel is slower (three cells a
+//     side 16 / 13; 4096 points at 3.2 F64 18 / 16; 10,000 at 2.4 15.7 / 17.0, at 3.2 18 / 21; 40,000 18 / 16,
+//     18 / 18, at 3.2 19 / 21; 90,000 31 / 18, 29 / 22, 31 / 29);
+//   * counting an undeformed lattice whose search radius is a lattice distance (r = 3 spacings: 128^3
+//     F32 267 -> 400 us, F64 450 -> 467, 64^3 55 -> 61 and 79 -> 72; a quarter of the neighbours are
+//     ties, each tested exactly): the list builder, which such clouds mostly go to, counts by cells.
 template <class F>
-bool runs_apply(const pn_grid& g, int64_t n) {
+bool runs_apply(const pn_grid& g, int64_t n, const CloudCells& cells) {
     if ((g.algorithm != 0 && !g.geom.periodic) || g.geom.hash || F::kFill) return false;
     if (g.grid.cap > (int64_t)1 << 28) return false;
-    if (8 * n < g.grid.n_sel) return false;
-    if (!F::kLight && g.nd == 2 && n < 32768 && !g.geom.periodic) return false;
+    if (6 * n < g.grid.n_sel) return false;
+    if (cells.in_octet > 0.0 && n >= (F::kLight ? 32768 : 8192) &&
+        cells.in_octet < (n < 32768 ? 1.45 : (g.nd == 2 ? 1.3 : 1.2)))
+        return false;
+    if (!F::kLight && g.nd == 2) {
+        const double per_cell = cells.per_cell;
+        if (g.geom.periodic) {
+            if (n >= 8192 && n < (per_cell < 5.5 ? 0 : (per_cell < 9 ? 32768 : 65536))) return false;
+        } else {
+            if (n < (per_cell < 5.5 ? 32768 : (per_cell < 9 ? 65536 : 262144))) return false;
+        }
+    }
     if (!(g.radius >= 0x1p-60 && g.radius <= 0x1p60)) return false;
     if (g.geom.periodic)
         for (int d = 0; d < g.nd; ++d)
@@ -591,7 +625,8 @@ bool runs_apply(const pn_grid& g, int64_t n) {
 // count 9.6 / 9.8 / 10.8 at 4096, 14.7 / 12.2 / 12.2 at 32,768, 104 / 62 / 43 at 512,000.  Queries that
 // are sparser than the grid's points have more candidates per run, so more work in each: they count
 // as fewer (100,000 probes among 512,000 bodies: n-body 87 / 68 / 86 us).
-void run_params(const pn_grid& g, int64_t n, int64_t n_sel, bool light, pn::RunScale& sc, pn::RunSplit& sp) {
+void run_params(const pn_grid& g, int64_t n, const CloudCells& cells, int64_t n_sel, bool light, pn::RunScale& sc,
+                pn::RunSplit& sp) {
     const pn::Geom& geom = g.geom;
     const double radius = g.radius;
     sc = pn::RunScale{};
@@ -608,6 +643,16 @@ void run_params(const pn_grid& g, int64_t n, int64_t n_sel, bool light, pn::RunS
     // 13.1 / 11.8, density 18.2 / 17.0, interact! 26.2 / 22.3; 1000 points 16.8 / 14.0 and 24.5 / 19.7;
     // 13,824 points 20.2 / 23.6 and 30.0 / 33.2).
     sp.lg_parts = (n + sp.most - 1) / sp.most <= 576 ? 1 : 0;
+    // A window of a sparse cloud, or of the sparse layer at the end of one that the cells cut thin, is many
+    // runs of a point or two, one after another: shorter windows and two wavefronts for each (uniform
+    // points, whole calls, us, as above / as here at .1, .3 and .6 a cell, which are 1.4, 2.3 and 3.6 filled
+    // cells in an octet: 100,000 points count 42 / 38, 28 / 23, 42 / 19, density 55 / 47, 39 / 29, 56 / 23;
+    // 20,000 points 24 / 15, 15 / 10, 15 / 10 and 24 / 20, 21 / 14, 21 / 14; at 1 a cell, 5.1, and with
+    // 500,000 points the windows above are better).
+    if (cells.in_octet > 0.0 && cells.in_octet < 4.3 && n <= 131072) {
+        sp.most = n <= 32768 ? 8 : 16;
+        sp.lg_parts = 1;
+    }
     sp.span = pn::RUN_SPAN;
     sp.magic0 = 0xffffffffu / (unsigned)geom.n[0];
     sp.magic1 = 0xffffffffu / (unsigned)geom.n[1];
@@ -638,7 +683,7 @@ int launch_runs(pn_grid& g, const BinSet* Q, const F& f) {
     const TR r = (TR)g.radius, r2 = r * r;
     pn::RunScale sc;
     pn::RunSplit sp;
-    run_params(g, n, Q->n_sel, F::kLight, sc, sp);
+    run_params(g, n, CloudCells(*Q), Q->n_sel, F::kLight, sc, sp);
     const int nblocks = (int)std::min<int64_t>(run_blocks(sp), g.persist_blocks);
     g.last_traversal = PN_TRAVERSAL_RUNS;
     LaunchTimer timer(g);  // brackets the one traversal kernel launched below
@@ -677,7 +722,8 @@ int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* 
         f.fstride = stride;
     }
     if constexpr (!F::kFill) {
-        if (allow_runs && runs_apply<F>(g, Q->stats_known ? Q->stats.n_binned : Q->n_sel)) return launch_runs<D, TC, TR, F>(g, Q, f);
+        if (allow_runs && runs_apply<F>(g, Q->stats_known ? Q->stats.n_binned : Q->n_sel, CloudCells(*Q)))
+            return launch_runs<D, TC, TR, F>(g, Q, f);
     }
     // Upper bound on non-empty query cells; the kernel reads the exact count on device.
     int64_t nwork = std::min<int64_t>(g.geom.ncells, Q->n_sel);

@@ -47,13 +47,37 @@ def test_knobs(chunk):
     assert density(nhs, x, x) == ("slices (large chunks)" if chunk == 1 else "slices")
 
 
-@pytest.mark.parametrize("n,want", [(32767, "cells"), (32768, "runs")])
-def test_2d(n, want):
-    nhs, x = search(2, n, 5.0)
+@pytest.mark.parametrize("n,a_cell,want", [(32767, 5.0, "cells"), (32768, 5.0, "runs"), (65535, 8.0, "cells"),
+                                           (65536, 8.0, "runs"), (262143, 11.0, "cells"), (262144, 11.0, "runs")])
+def test_2d(n, a_cell, want):
+    nhs, x = search(2, n, a_cell)
     assert density(nhs, x, x) == want and count(nhs, x, x) == "runs"
 
 
-@pytest.mark.parametrize("n_x,want", [(9999, "cells"), (10000, "runs")])
+@pytest.mark.parametrize("side,r,want", [(90, 3.2, "runs"), (91, 3.2, "cells"), (91, 2.0, "runs"), (181, 2.6, "cells"),
+                                         (182, 2.6, "runs"), (255, 3.2, "cells"), (256, 3.2, "runs")])
+def test_2d_periodic(side, r, want):
+    from test_gpu_parity import dev
+    pts = (np.stack(np.meshgrid(*[np.arange(side)] * 2, indexing="ij"), -1).reshape(-1, 2) + 0.5).astype(np.float32)
+    size = np.full(2, side, np.float32)
+    box = pn.PeriodicBox(min_corner=np.zeros(2, np.float32), max_corner=size)
+    cl = pn.FullGridCellList(min_corner=box.min_corner, max_corner=box.max_corner, search_radius=np.float32(r))
+    nhs = pn.GridNeighborhoodSearch[2](search_radius=np.float32(r), n_points=len(pts), periodic_box=box, cell_list=cl)
+    x = dev(pts)
+    pn.initialize(nhs, x, x)
+    assert density(nhs, x, x) == want and count(nhs, x, x) == "runs"
+
+
+@pytest.mark.parametrize("D,n,a_cell,kinds", [(3, 100_000, 0.02, "cells cells"), (3, 100_000, 0.2, "runs runs"),
+                                              (2, 100_000, 0.05, "cells cells"), (2, 100_000, 0.2, "runs runs"),
+                                              (3, 20_000, 0.05, "runs cells"), (3, 20_000, 0.3, "runs runs"),
+                                              (3, 8000, 0.02, "runs runs")])
+def test_sparse_clouds(D, n, a_cell, kinds):
+    nhs, x = search(D, n, a_cell)
+    assert [count(nhs, x, x), density(nhs, x, x)] == kinds.split()
+
+
+@pytest.mark.parametrize("n_x,want", [(13333, "cells"), (13334, "runs")])
 def test_sparse_queries(n_x, want):
     nhs, y = search(3, 80_000, 10.0)
     x = y[:, :n_x].t().contiguous().t()
