@@ -66,7 +66,7 @@ struct RunSplit {
     int n;     // points that the host expects; the kernels read their number on the device
     int most;  // queries of a run, a power of two up to RUN
     int lg_parts;  // 2^lg_parts wavefronts share the runs of a window of `most` positions
-    int span;  // cells of a run (one where the coordinates moved since the binning)
+    int span;  // cells of a run
     unsigned magic0, magic1;  // floor((2^32 - 1) / cells) in x and y (no batch table)
     int cell64;  // cells are computed in Float64
 };
@@ -131,15 +131,17 @@ __device__ __forceinline__ void for_windows(int n, int nblocks, const RunSplit& 
 
 // Calls fn(RunDesc) for the runs of window w that are this part's, every 2^lg_parts-th: the window of
 // `most` (at most RUN) sorted positions is cut where the x-row changes, where a run would cover more
-// than `span` cells and at gaps.
+// than `span` cells (one where the coordinates moved since the binning) and at gaps.
 template <int D, class Fn>
-__device__ __forceinline__ void for_runs(const Geom& g, const SetView& Q, int w, int part, int n, const RunSplit& sp,
-                                         Fn&& fn) {
+__device__ __forceinline__ void for_runs(const Geom& g, const SetView& Q, int w, int part, int n, int moved,
+                                         const RunSplit& sp, Fn&& fn) {
     const int lane = threadIdx.x;
     const int p0 = w * sp.most, mask = (1 << sp.lg_parts) - 1;
     int turn = part;
     const int key_l = Q.keys[min((int64_t)p0 + lane, Q.cap - 1)];  // lanes from cnt on are not looked at
     const int cnt = min(sp.most, n - p0);
+    asm volatile("" : "+s"(moved));  // not waited for before the keys are on their way
+    const int span = moved ? 1 : sp.span;
     const int step = key_l - __shfl_up(key_l, 1, WAVE);
     RunDesc rd;
     rd.n0 = g.n[0];
@@ -167,7 +169,7 @@ __device__ __forceinline__ void for_runs(const Geom& g, const SetView& Q, int w,
         rd.cy = (int)yz - rd.cz * rd.n1;
         const int cx = key_l - rd.row;
         rd.ca = key - rd.row;
-        const bool cut = lane > i && (lane >= cnt || cx >= min(rd.n0, rd.ca + sp.span) || step >= RUN_GAP);
+        const bool cut = lane > i && (lane >= cnt || cx >= min(rd.n0, rd.ca + span) || step >= RUN_GAP);
         const int end = __builtin_ctzll(__builtin_amdgcn_ballot_w64(cut));  // cnt < 64 at the latest
         rd.q0 = p0 + i;
         rd.nq = end - i;
@@ -532,10 +534,9 @@ __global__ __launch_bounds__(WAVE, 4) void k_runs_count(Geom g, SetView Q, SetVi
 #pragma unroll
     for (int d = 0; d < D; ++d) box[d] = (TR)g.box[d];
     const TR r2_in = r2 - r2 * (TR)sc.cell_rel;  // up to this x distance squared cells are adjacent
-    const int n = Q.st->n_binned;
-    if (Gs.st->moved) sp.span = 1;
+    const int n = Q.st->n_binned, moved = Gs.st->moved;
     for_windows(n, nblocks, sp, [&](int w, int part) {
-        for_runs<D>(g, Q, w, part, n, sp, [&](const RunDesc& rd) {
+        for_runs<D>(g, Q, w, part, n, moved, sp, [&](const RunDesc& rd) {
             const RunLanes ln(rd.nq);
             const bool qact = ln.query < rd.nq;
             const int qpos = rd.q0 + (qact ? ln.query : 0);
@@ -721,10 +722,9 @@ __global__ __launch_bounds__(WAVE, (sizeof(TR) == 8 ? 3 : 4)) void k_runs(Geom g
 #pragma unroll
     for (int d = 0; d < D; ++d) box[d] = (TR)g.box[d];
     const TR r2_in = r2 - r2 * (TR)sc.cell_rel;  // up to this x distance squared cells are adjacent
-    const int n = Q.st->n_binned;
-    if (Gs.st->moved) sp.span = 1;
+    const int n = Q.st->n_binned, moved = Gs.st->moved;
     for_windows(n, nblocks, sp, [&](int w, int part) {
-        for_runs<D>(g, Q, w, part, n, sp, [&](const RunDesc& rd) {
+        for_runs<D>(g, Q, w, part, n, moved, sp, [&](const RunDesc& rd) {
             const RunLanes ln(rd.nq);
             const bool qact = ln.query < rd.nq;
             const int qpos = rd.q0 + (qact ? ln.query : 0);
