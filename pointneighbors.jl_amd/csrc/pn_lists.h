@@ -731,8 +731,8 @@ __device__ __forceinline__ void load_rec(const uint4* __restrict__ rec, int64_t 
 
 // k_list_tlsph_force<D, T, K, true> over packed records (same terms, same operation order, so
 // the same bits); one neighbour in flight per lane, which measured fastest with the wide loads
-// (its record fills the registers).  The gathers bound it: 117 neighbours times 128 bytes for
-// each of 101^3 points are 15 GB through the caches.  The next neighbour's list entry is loaded
+// (its record fills the registers).  The gathers bound it: 105 neighbours times 112 bytes for
+// each of 101^3 points are 12 GB through the caches.  The next neighbour's list entry is loaded
 // before this one's arithmetic, so that a step waits for one load and not for two in a row, and
 // larger workgroups share more lines (ListShape): pack included, Float32 927 -> 821 us, Float64
 // 1740 -> 1643 us.  Gathering whole records into LDS took 849 us and more (Float64 2.1 ms), one
