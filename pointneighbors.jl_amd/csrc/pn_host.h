@@ -679,7 +679,6 @@ int64_t run_blocks(const pn::RunSplit& sp) { return round_up8((sp.n + sp.most - 
 template <int D, class TC, class TR, class F>
 int launch_runs(pn_grid& g, const BinSet* Q, const F& f) {
     const int64_t n = Q->stats_known ? Q->stats.n_binned : Q->n_sel;
-    if (n == 0) return PN_OK;
     const TR r = (TR)g.radius, r2 = r * r;
     pn::RunScale sc;
     pn::RunSplit sp;
@@ -728,8 +727,8 @@ int launch_traverse_t(pn_grid& g, const BinSet* Q, F f, const pn::FieldSrc<TR>* 
     // Upper bound on non-empty query cells; the kernel reads the exact count on device.
     int64_t nwork = std::min<int64_t>(g.geom.ncells, Q->n_sel);
     if (Q->stats_known) nwork = Q->stats.n_nonempty;
-    if (nwork == 0) return PN_OK;
-    const int nblocks = (int)std::min<int64_t>(round_up8(nwork), g.persist_blocks);
+    // at least a workgroup for each XCD: a replayed binning may have filled cells since
+    const int nblocks = (int)std::min<int64_t>(round_up8(std::max<int64_t>(nwork, 1)), g.persist_blocks);
     const TR r = (TR)g.radius;
     const TR r2 = r * r;
     LaunchTimer timer(g);  // brackets the one traversal kernel launched below

@@ -107,8 +107,10 @@ __device__ __forceinline__ unsigned div_magic(unsigned x, unsigned n, unsigned m
 // slowest dimension, and one that the cells cut thin has few points a row: its runs cover up to 32
 // cells and take some times as long as others, and started last they kept the chip waiting (us, all
 // ascending / as here, lattices whose last layer is thin: 512,000 points at r = 2.4 spacings count
-// 100 / 69, density 153 / 97; 1 M at 3.2 count 236 / 146, density 401 / 276, interact! 626 / 448; without
-// such a layer the same).
+// 100 / 69, density 153 / 97; 1 M at 3.2 count 236 / 146, density 401 / 276, interact! 626 / 448).  Other
+// clouds lose 1 to 2 % to the scalar registers that this and the device's number of points take (1.14 M
+// points in 64 clouds count 116 / 118, 1 M points density 161 / 162, pressure 188 / 190; all of it computed
+// again for each window instead: more spills).
 // sp.n shares the windows out, so that no load waits for n, the number of points on the device (0.3 us
 // of a launch); where n is larger, the windows behind follow in turn.
 template <class Fn>

@@ -84,3 +84,30 @@ def test_more_points_than_the_host_knows(n, fewer):
     check(load().pn_sum_neighbor_indices(nhs._handle, PN_QUERIES_GRID, ctypes.c_void_p(sums.data_ptr()), 0, 0))
     assert np.array_equal(counts.cpu().numpy(), gpu_counts(plain, x, x))
     assert np.array_equal(sums.cpu().numpy(), gpu_sums(plain, x, x))
+
+
+@pytest.mark.parametrize("algorithm", [0, 1])
+@pytest.mark.parametrize("D", [1, 3])
+def test_host_knows_of_an_empty_binning(D, algorithm):
+    """The host has read the status of a replay that dropped every point; the next one bins them all."""
+    from test_gpu_parity import dev, gpu_counts, make_nhs
+    n = 700
+    pts = np.random.default_rng(n).uniform(0.0, 5.0, (n, D)).astype(np.float32)
+    nhs, plain = (make_nhs(pts, np.float32(1.0), pts.min(axis=0) - 3, pts.max(axis=0) + 3, cap=1000) for _ in range(2))
+    x, y = dev(pts), dev(pts)
+    pn.initialize(nhs, x, x)
+    pn.initialize(plain, y, y)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        pn.update(nhs, x, x, check_errors=False)
+    nhs._set_stream(x)
+    x.fill_(float("nan"))
+    graph.replay()
+    assert nhs.stats()[0] == 0
+    x.copy_(y)
+    graph.replay()
+    nhs.set_tuning("algorithm", algorithm)
+    counts = torch.full((n,), UNTOUCHED, dtype=torch.int32, device="cuda")
+    check(load().pn_count_neighbors(nhs._handle, PN_QUERIES_GRID, ctypes.c_void_p(counts.data_ptr()), 0))
+    assert np.array_equal(counts.cpu().numpy(), gpu_counts(plain, y, y))
